@@ -268,9 +268,13 @@ int amr_dev_stage(amr_dev *dev, int start, int num, int stage, int permute,
  * variables; set_mesh, split, consolidate, stencil, download_block, the
  * halo codec and save_state first bring them up to date (to the values
  * amr_dev_stage would have written, from the interiors the stage read).
- * It is amr_dev_stage without two interiors, with permute != 0, while the
- * tape records, and for stages of fewer than 1e8 cell updates
- * (latency-bound; MINIAMR_FUSED=2 at creation fuses those too). */
+ * With the 7-point stencil every ghost plane -- boundary and coarse/fine ones
+ * too -- is read from where its values come from, at any stage size and
+ * with permute, where the block's ghost box fits in LDS.  It is
+ * amr_dev_stage without two interiors, with permute != 0, while the tape
+ * records, when the jobs name blocks outside the active list, and for
+ * stages of fewer than 1e8 cell updates (latency-bound; MINIAMR_FUSED=2 at
+ * creation fuses those too). */
 int amr_dev_stage_fused(amr_dev *dev, int start, int num, int stage, int permute,
                         int sum_row);
 

@@ -986,6 +986,8 @@ int amr_dev_save_state(amr_dev *d, void *dst)
    size_t bytes = 0;
    if (!d || !dst || amr_dev_state_bytes(d, &bytes))
       return amr_set_error(d, AMR_ERR_ARG, "save_state: bad arguments");
+   if (int rc = amr_home_copies(d))   // a saved state holds its cells in the first copy
+      return rc;
    HIP_TRY(d, hipMemcpyAsync(dst, d->pool, bytes, hipMemcpyDefault, d->stream));
    HIP_TRY(d, hipStreamSynchronize(d->stream));
    return AMR_OK;
@@ -996,6 +998,9 @@ int amr_dev_load_state(amr_dev *d, const void *src)
    size_t bytes = 0;
    if (!d || !src || amr_dev_state_bytes(d, &bytes))
       return amr_set_error(d, AMR_ERR_ARG, "load_state: bad arguments");
+   std::fill(d->par.begin(), d->par.end(), 0);   // as save_state left it
+   std::fill(d->slot_par.begin(), d->slot_par.end(), 0);
+   std::fill(d->stale.begin(), d->stale.end(), 0);
    HIP_TRY(d, hipStreamSynchronize(d->stream));
    HIP_TRY(d, hipMemcpyAsync(d->pool, src, bytes, hipMemcpyDefault, d->stream));
    HIP_TRY(d, hipStreamSynchronize(d->stream));

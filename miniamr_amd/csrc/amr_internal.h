@@ -87,6 +87,19 @@ __host__ __device__ __forceinline__ int64_t edge_at(const EdgeSrc &e, const Lay 
    return (int64_t) e.slot * L.rec + e.off + part + (int64_t) t * e.stride;
 }
 
+// Where a stage that reads faces in place finds the ghost plane of one face
+// of an active block (six entries per block, sorted order).  FS_OWN: the
+// block's own ghost plane.  FS_SAME: the interior plane of the same-level
+// neighbour s[0].  FS_BC: the block's own plane next to the domain boundary.
+// FS_PROLONG: quarter (iq, jq) = (s[1], s[2]) of the coarse neighbour s[0]'s
+// plane, divided by 4.  FS_RESTRICT: sums of four cells of the fine
+// neighbours s[iq + 2*jq] (-1: no job fills that quarter).
+enum { FS_OWN = 0, FS_SAME = 1, FS_BC = 2, FS_PROLONG = 3, FS_RESTRICT = 4 };
+struct FaceSrc {
+   int32_t kind;
+   int32_t s[4];
+};
+
 // Recorded data operations of a context (include/amr_adjoint.h): each op
 // is {kind, args..., plan in force}; plans and job lists are host copies.
 struct TapePlan {
@@ -211,6 +224,20 @@ struct amr_dev {
    std::vector<Span> spans;
 
    char err[512] = {0};
+
+   // The faces of each active block (six FaceSrc, sorted order).  all_faces:
+   // a 7-point stage reads every face in place (each ghost plane has one
+   // same-level, boundary or coarse/fine source and all blocks the jobs
+   // name are active), so it needs no exchange at all.
+   FaceSrc *d_faces = nullptr;
+   bool all_faces = false;
+   // closed: every block the plan's jobs name is active, so all of them hold
+   // their cells in the copy par names (a fused stage needs that)
+   bool closed = false;
+   // The copy that holds an inactive slot's cells: par as it was when the
+   // slot was last written or active ([slot][variable]; two interiors only).
+   std::vector<uint8_t> slot_par;
+   std::vector<uint8_t> active;     // per slot: in the active list (two interiors only)
 };
 
 // Storage helpers: T is double, float or uint16_t (bfloat16 bits); A is the
@@ -237,6 +264,11 @@ template <> __device__ __forceinline__ uint16_t from_acc<uint16_t>(float v)
    u += 0x7fffu + ((u >> 16) & 1u);
    return (uint16_t) (u >> 16);
 }
+
+// C adjacent cells as one vector.
+template <typename T, int C> struct VecN {
+   typedef T __attribute__((ext_vector_type(C))) type;
+};
 
 // Global-memory view of a device pointer.  A pointer that a kernel reads
 // from memory (the batch's item records) is otherwise a generic address,
@@ -429,10 +461,30 @@ int amr_lay(amr_dev *d, int start, int num, Lay *out);
 // The same layout with the other interior copy (where a stage writes).
 Lay amr_lay_other(const amr_dev *d, const Lay &L);
 
+// Bring the cells of inactive slots among slots[0..n) to the copy par names
+// (they stay behind when fused stages move the active blocks' cells).
+int amr_slots_current(amr_dev *d, const int32_t *slots, int n);
+bool amr_slot_current(const amr_dev *d, int slot);
+// The same for what split jobs read; their children are written whole.
+int amr_split_slots_current(amr_dev *d, const amr_split_job *jobs, int n);
+// All cells to the first interior copy, par included: the form of a saved
+// state, whatever stages ran before.
+int amr_home_copies(amr_dev *d);
+// Slot `slot` was written in the copy par names.
+void amr_slot_written(amr_dev *d, int slot);
+
 // Launchers implemented per source file; all enqueue on d->stream.
 int amr_launch_exchange_dir(amr_dev *d, int dir, int start, int num);
 int amr_launch_exchange_fused_dir(amr_dev *d, int dir, int start, int num);
 int amr_launch_stencil(amr_dev *d, int start, int num, bool want_partials, int calc_stage);
+// The whole-box stencil (box.hip; st: 7 or 27) where the block's ghost box fits
+// in LDS: interiors read in copy L and written in copy Lo, face ghosts where
+// faces says (null: the block's own ghost planes), 27-point edges where edges
+// says (null: its own).
+bool amr_box_fits(const amr_dev *d, int st);
+bool amr_uses_box(const amr_dev *d);   // the context's 7- or 27-point stencil is a box one
+int amr_launch_box(amr_dev *d, int st, const FaceSrc *faces, const EdgeSrc *edges, const Lay &L,
+                   const Lay &Lo, int start, int num, double *parts);
 int amr_launch_mat_stencil(amr_dev *d, int var, int calc_stage);
 // Stencil of a fused stage: interiors read from the current copy, written
 // to the other one (the variables' copy flips), same-level faces read in

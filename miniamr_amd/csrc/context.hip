@@ -6,6 +6,7 @@
 #include <string.h>
 #include <algorithm>
 #include <thread>
+#include <type_traits>
 
 #include "amr_adjoint.h"
 #include "amr_internal.h"
@@ -116,6 +117,10 @@ int amr_dev_create(const amr_dev_config *cfg, amr_dev **out)
    }
    d->par.assign(cfg->num_vars, 0);
    d->stale.assign(cfg->num_vars, 0);
+   if (d->two_interiors) {
+      d->slot_par.assign((size_t) cfg->num_vars * cfg->max_blocks, 0);
+      d->active.assign(cfg->max_blocks, 0);
+   }
    int64_t cells = (int64_t) g.gx * g.gy * g.gz;
    g.var_stride = g.rec * cfg->max_blocks;
    size_t pool_bytes = (size_t) g.var_stride * cfg->num_vars * d->elem_bytes;
@@ -161,6 +166,7 @@ int amr_dev_destroy(amr_dev *d)
    hipFree(d->d_cmp);
    hipFree(d->d_fjobs);
    hipFree(d->d_redir);
+   hipFree(d->d_faces);
    hipFree(d->d_edges);
    hipFree(d->d_mjobs);
    hipFree(d->d_a0);
@@ -201,6 +207,7 @@ int amr_dev_upload_block(amr_dev *d, int slot, const double *cells)
    if (rc)
       return rc;
    HIP_TRY(d, hipStreamSynchronize(d->stream));
+   amr_slot_written(d, slot);
    amr_tape_record(d, AMR_OP_UPLOAD, slot);
    return AMR_OK;
 }
@@ -211,6 +218,8 @@ int amr_dev_download_block(amr_dev *d, int slot, double *cells)
       return AMR_ERR_STATE;
    if (!d || !cells || slot < 0 || slot >= d->c.max_blocks)
       return amr_set_error(d, AMR_ERR_ARG, "download: slot %d out of range", slot);
+   if (int rc = amr_slots_current(d, &slot, 1))
+      return rc;
    int rc = amr_launch_convert_out(d, slot);
    if (rc)
       return rc;
@@ -245,6 +254,116 @@ Lay amr_lay_other(const amr_dev *d, const Lay &L)
    o.oI = d->oI_par[1 - p];
    o.oZI = d->oZI_par[1 - p];
    return o;
+}
+
+// ---- inactive slots and the two interior copies
+// A fused stage moves the cells of the active blocks from one interior copy
+// to the other; a slot outside the active list keeps its cells where they
+// were written.  slot_par remembers that copy, and whatever looks at such a
+// slot (a download, the codec, a split or consolidation, a mesh that makes
+// it active or reads it) first has its interior and z-plane copies moved.
+// The moves travel as kernel arguments: no allocation, nothing to wait for.
+struct CopyMove {
+   int32_t slot, var, num, from;   // variables [var, var+num), from copy `from`
+};
+constexpr int kMoves = 64;
+struct CopyMoves {
+   CopyMove m[kMoves];
+};
+
+template <typename T>
+static __global__ void k_move_copies(T *__restrict__ pool, CopyMoves mv, Lay L, int4 off, int nI,
+                                     int nZ)
+{
+   const CopyMove m = mv.m[blockIdx.x];
+   if ((int) blockIdx.y >= m.num)
+      return;
+   T *rec = pool + (int64_t) (m.var + blockIdx.y) * L.var_stride + (int64_t) m.slot * L.rec;
+   const int sI = m.from ? off.y : off.x, dI = m.from ? off.x : off.y;
+   const int sZ = m.from ? off.w : off.z, dZ = m.from ? off.z : off.w;
+   for (int t = threadIdx.x; t < nI; t += blockDim.x)
+      rec[dI + t] = rec[sI + t];
+   for (int t = threadIdx.x; t < nZ; t += blockDim.x)
+      rec[dZ + t] = rec[sZ + t];
+}
+
+static int move_copies(amr_dev *d, const std::vector<CopyMove> &mv)
+{
+   const int4 off = make_int4(d->oI_par[0], d->oI_par[1], d->oZI_par[0], d->oZI_par[1]);
+   const int nI = d->g.nx * d->g.ny * d->g.nz, nZ = 2 * d->g.nx * d->g.ny;
+   for (size_t t = 0; t < mv.size(); t += kMoves) {
+      CopyMoves a;
+      const int n = (int) std::min<size_t>(kMoves, mv.size() - t);
+      memset(&a, 0, sizeof(a));
+      memcpy(a.m, &mv[t], sizeof(CopyMove) * n);
+      const dim3 grid(n, d->c.num_vars);
+      if (d->elem_bytes == 8)
+         hipLaunchKernelGGL(k_move_copies<uint64_t>, grid, dim3(256), 0, d->stream,
+                            (uint64_t *) d->pool, a, d->g, off, nI, nZ);
+      else if (d->elem_bytes == 4)
+         hipLaunchKernelGGL(k_move_copies<uint32_t>, grid, dim3(256), 0, d->stream,
+                            (uint32_t *) d->pool, a, d->g, off, nI, nZ);
+      else
+         hipLaunchKernelGGL(k_move_copies<uint16_t>, grid, dim3(256), 0, d->stream,
+                            (uint16_t *) d->pool, a, d->g, off, nI, nZ);
+      HIP_TRY(d, hipGetLastError());
+   }
+   return AMR_OK;
+}
+
+// The moves that bring slot `slot`, held as `is` says, to the copies `want`.
+static void add_moves(std::vector<CopyMove> &mv, int slot, const uint8_t *is, const uint8_t *want,
+                      int nv)
+{
+   for (int v = 0; v < nv;) {
+      int e = v + 1;
+      while (e < nv && is[e] == is[v] && want[e] == want[v])
+         e++;
+      if (is[v] != want[v])
+         mv.push_back({slot, v, e - v, is[v]});
+      v = e;
+   }
+}
+
+void amr_slot_written(amr_dev *d, int slot)
+{
+   if (d->two_interiors)
+      memcpy(&d->slot_par[(size_t) slot * d->c.num_vars], d->par.data(), d->c.num_vars);
+}
+
+bool amr_slot_current(const amr_dev *d, int slot)
+{
+   return !d->two_interiors || d->active[slot] ||
+          !memcmp(&d->slot_par[(size_t) slot * d->c.num_vars], d->par.data(), d->c.num_vars);
+}
+
+int amr_slots_current(amr_dev *d, const int32_t *slots, int n)
+{
+   std::vector<CopyMove> mv;
+   for (int t = 0; t < n; t++)
+      if (!amr_slot_current(d, slots[t])) {
+         add_moves(mv, slots[t], &d->slot_par[(size_t) slots[t] * d->c.num_vars], d->par.data(),
+                   d->c.num_vars);
+         amr_slot_written(d, slots[t]);
+      }
+   return move_copies(d, mv);
+}
+
+int amr_home_copies(amr_dev *d)
+{
+   if (!d->two_interiors)
+      return AMR_OK;
+   for (int s : d->h_sorted)
+      amr_slot_written(d, s);
+   const std::vector<uint8_t> home(d->c.num_vars, 0);
+   std::vector<CopyMove> mv;
+   for (int s = 0; s < d->c.max_blocks; s++)
+      add_moves(mv, s, &d->slot_par[(size_t) s * d->c.num_vars], home.data(), d->c.num_vars);
+   if (int rc = move_copies(d, mv))
+      return rc;
+   std::fill(d->slot_par.begin(), d->slot_par.end(), 0);
+   std::fill(d->par.begin(), d->par.end(), 0);
+   return AMR_OK;
 }
 
 // MINIAMR_HOIST=0 keeps every fused job in its own direction's launch (the
@@ -419,10 +538,65 @@ struct FusedPlan {
    int32_t fc[3] = {0, 0, 0};
    std::vector<EdgeSrc> edges;
    std::vector<int32_t> redir;
+   std::vector<FaceSrc> faces;
+   bool all_faces = false;
    std::vector<amr_face_job> mj;
    int32_t mc[3] = {0, 0, 0};
    bool fold = false;
 };
+
+// The plan's FaceSrc table.  27-point stencil: the faces read in place (same
+// level) and the block's own planes.  7-point stencil: every face in place
+// when that is possible (all_faces): its jobs read interiors only, at every
+// kind, so no ghost plane is needed as long as each has at most one source
+// (four quarters for a restriction) and all blocks named are active.  Empty
+// where the plane-by-plane kernels serve.
+static void face_sources(const amr_dev *d, const int32_t *sorted, int n_active,
+                         const amr_face_job *jobs, int nj, FusedPlan &P)
+{
+   P.all_faces = false;
+   P.faces.clear();
+   if (!amr_uses_box(d))
+      return;
+   if (d->g.stencil != 7) {
+      P.faces.assign(6 * (size_t) n_active, FaceSrc{FS_OWN, {-1, -1, -1, -1}});
+      for (size_t i = 0; i < 6 * (size_t) n_active; i++)
+         if (P.redir[i] >= 0)
+            P.faces[i] = FaceSrc{FS_SAME, {P.redir[i], -1, -1, -1}};
+      return;
+   }
+   std::vector<int32_t> at(d->c.max_blocks, -1);   // slot -> place in sorted
+   bool ok = true;
+   for (int in = 0; in < n_active; in++) {
+      ok &= at[sorted[in]] < 0;
+      at[sorted[in]] = in;
+   }
+   std::vector<FaceSrc> F(6 * (size_t) std::max(n_active, 1), FaceSrc{FS_OWN, {-1, -1, -1, -1}});
+   for (int t = 0; t < nj && ok; t++) {
+      const amr_face_job &j = jobs[t];
+      ok = at[j.dst] >= 0 && at[j.src] >= 0 && !(j.kind & AMR_FACE_GHOSTS);
+      if (!ok)
+         break;
+      FaceSrc &f = F[6 * (size_t) at[j.dst] + j.face];
+      if (j.kind == AMR_FACE_RESTRICT) {
+         int32_t &q = f.s[j.iq + 2 * j.jq];
+         ok = (f.kind == FS_OWN || f.kind == FS_RESTRICT) && q < 0;
+         f.kind = FS_RESTRICT;
+         q = j.src;
+      } else {
+         ok = f.kind == FS_OWN;
+         if (j.kind == AMR_FACE_SAME) f = FaceSrc{FS_SAME, {j.src, -1, -1, -1}};
+         else if (j.kind == AMR_FACE_BC) f = FaceSrc{FS_BC, {-1, -1, -1, -1}};
+         else f = FaceSrc{FS_PROLONG, {j.src, j.iq, j.jq, -1}};
+      }
+   }
+   P.all_faces = ok;
+   if (!ok)   // the other fused stage: same-level faces in place
+      for (size_t i = 0; i < 6 * (size_t) n_active; i++)
+         F[i] = P.redir[i] >= 0 ? FaceSrc{FS_SAME, {P.redir[i], -1, -1, -1}}
+                                : FaceSrc{FS_OWN, {-1, -1, -1, -1}};
+   P.faces.swap(F);
+}
 
 static void compute_fused_plan(const amr_dev *d, const int32_t *sorted, int n_active,
                                const amr_face_job *jobs, const int32_t count[3], FusedPlan &P)
@@ -533,6 +707,7 @@ static void compute_fused_plan(const amr_dev *d, const int32_t *sorted, int n_ac
    for (int in = 0; in < n_active; in++)
       for (int f = 0; f < 6; f++)
          P.redir[6 * (size_t) in + f] = inplace(sorted[in], f);
+   face_sources(d, sorted, n_active, jobs, nj, P);
 }
 
 // A fused stage leaves unwritten the ghost cells its stencil reads where
@@ -560,8 +735,11 @@ int amr_require_fresh(amr_dev *d, int start, int num, const char *what)
       if (int rc = amr_lay(d, a, b - a, &L))
          return rc;
       const Lay Lr = amr_lay_other(d, L);
-      for (int dir = 0, off = 0; dir < 3; off += d->mcount[dir], dir++)
-         if (int rc = amr_launch_exchange_jobs(d, d->d_mjobs + off, d->mcount[dir], Lr, a, b - a))
+      // a stage that read every face in place left every ghost plane
+      const amr_face_job *jobs = d->all_faces ? d->d_jobs : d->d_mjobs;
+      const int32_t *cnt = d->all_faces ? d->count : d->mcount;
+      for (int dir = 0, off = 0; dir < 3; off += cnt[dir], dir++)
+         if (int rc = amr_launch_exchange_jobs(d, jobs + off, cnt[dir], Lr, a, b - a))
             return amr_set_error(d, rc, "%s: bringing ghost planes up to date: %s", what,
                                  d->err);
       for (int v = a; v < b; v++)
@@ -599,6 +777,25 @@ int amr_set_mesh_impl(amr_dev *d, const int32_t *sorted, int n_active,
           j.src < 0 || j.src >= d->c.max_blocks || (j.iq & ~1) || (j.jq & ~1))
          return amr_set_error(d, AMR_ERR_ARG, "set_mesh: bad face job %d", t);
    }
+   if (d->two_interiors) {
+      for (int x : d->h_sorted) {   // slots that leave the list stay where they are
+         amr_slot_written(d, x);
+         d->active[x] = 0;
+      }
+      std::vector<int32_t> used(sorted, sorted + n_active);
+      std::vector<uint8_t> act(d->c.max_blocks, 0);
+      for (int i = 0; i < n_active; i++)
+         act[sorted[i]] = 1;
+      d->closed = true;
+      for (int t = 0; t < nj; t++) {
+         if (!act[jobs[t].src])
+            used.push_back(jobs[t].src);
+         d->closed &= act[jobs[t].src] && act[jobs[t].dst];
+      }
+      if (int rc = amr_slots_current(d, used.data(), (int) used.size()))
+         return rc;
+      d->active.swap(act);
+   }
    // The fused plan is host work; it runs before the wait below, so it
    // overlaps the device work still queued (split and consolidate data).
    FusedPlan fp;
@@ -630,6 +827,8 @@ int amr_set_mesh_impl(amr_dev *d, const int32_t *sorted, int n_active,
          HIP_TRY(d, hipMalloc(&d->d_edges, sizeof(EdgeSrc) * fp.edges.size()));
       if (!d->d_redir)
          HIP_TRY(d, hipMalloc(&d->d_redir, sizeof(int32_t) * 6 * (size_t) d->c.max_blocks));
+      if (!d->d_faces)
+         HIP_TRY(d, hipMalloc(&d->d_faces, sizeof(FaceSrc) * 6 * (size_t) d->c.max_blocks));
    }
    // One pinned staging buffer, then copies ordered on the stream before
    // any later launch (pageable hipMemcpy of the ~3 MB plan took 0.5-2 ms).
@@ -645,6 +844,7 @@ int amr_set_mesh_impl(amr_dev *d, const int32_t *sorted, int n_active,
       pieces.push_back({d->d_fjobs, fp.fj.data(), sizeof(FusedJob) * fp.fj.size()});
       pieces.push_back({d->d_edges, fp.edges.data(), sizeof(EdgeSrc) * fp.edges.size()});
       pieces.push_back({d->d_redir, fp.redir.data(), sizeof(int32_t) * fp.redir.size()});
+      pieces.push_back({d->d_faces, fp.faces.data(), sizeof(FaceSrc) * fp.faces.size()});
       pieces.push_back({d->d_mjobs, fp.mj.data(), sizeof(amr_face_job) * fp.mj.size()});
    }
    size_t total = 0;
@@ -677,6 +877,7 @@ int amr_set_mesh_impl(amr_dev *d, const int32_t *sorted, int n_active,
    d->plan_version++;
    if (d->two_interiors) {
       d->fold_edges = fp.fold;
+      d->all_faces = fp.all_faces;
       for (int i = 0; i < 3; i++) {
          d->fcount[i] = fp.fc[i];
          d->mcount[i] = fp.mc[i];
@@ -853,6 +1054,50 @@ static int ensure_jobbuf(amr_dev *d, size_t bytes)
    return AMR_OK;
 }
 
+// Jobs read slots where they are and write them where par says.  A slot that
+// is written whole (a child; a merged block by its eight octants) needs no
+// move of what it held.
+template <typename J>
+static int refine_slots_current(amr_dev *d, const J *jobs, int n)
+{
+   if (!d->two_interiors)
+      return AMR_OK;
+   std::vector<uint8_t> octants;   // of each merged block, when first needed
+   for (int t = 0; t < n; t++) {
+      int32_t rd, wr;
+      if constexpr (std::is_same<J, amr_split_job>::value) {
+         rd = jobs[t].parent;
+         wr = jobs[t].child;
+      } else {
+         rd = jobs[t].child;
+         wr = jobs[t].dst;
+      }
+      if (int rc = amr_slots_current(d, &rd, 1))
+         return rc;
+      if (amr_slot_current(d, wr))
+         continue;
+      if constexpr (!std::is_same<J, amr_split_job>::value) {
+         if (octants.empty()) {
+            octants.assign(d->c.max_blocks, 0);
+            for (int q = t; q < n; q++)
+               octants[jobs[q].dst] |= 1 << jobs[q].octant;
+         }
+         if (octants[wr] != 0xff) {
+            if (int rc = amr_slots_current(d, &wr, 1))
+               return rc;
+            continue;
+         }
+      }
+      amr_slot_written(d, wr);
+   }
+   return AMR_OK;
+}
+
+int amr_split_slots_current(amr_dev *d, const amr_split_job *jobs, int n)
+{
+   return refine_slots_current(d, jobs, n);
+}
+
 template <typename J>
 static int refine_data(amr_dev *d, const J *jobs, int n, bool split)
 {
@@ -870,6 +1115,8 @@ static int refine_data(amr_dev *d, const J *jobs, int n, bool split)
       if (a < 0 || a >= d->c.max_blocks || b < 0 || b >= d->c.max_blocks || o < 0 || o > 7)
          return amr_set_error(d, AMR_ERR_ARG, "split/consolidate: bad job %d", t);
    }
+   if (int rc = refine_slots_current(d, jobs, n))
+      return rc;
    size_t per_job = (size_t) d->c.num_vars * (d->g.nx / 2) * (d->g.ny / 2) * (d->g.nz / 2) *
                     d->elem_bytes;
    int chunk = (int) std::max<size_t>(1, std::min<size_t>(n, kScratchCap / per_job));
@@ -941,7 +1188,7 @@ extern "C" {
 
 int amr_dev_split(amr_dev *d, const amr_split_job *jobs, int n)
 {
-   int rc = refine_data(d, jobs, n, true);
+   int rc = amr_split_impl(d, jobs, n);
    if (!rc && n && d->tape && d->tape->on && !d->replaying) {
       const int first = (int) d->tape->splits.size();
       d->tape->splits.insert(d->tape->splits.end(), jobs, jobs + n);
@@ -952,7 +1199,7 @@ int amr_dev_split(amr_dev *d, const amr_split_job *jobs, int n)
 
 int amr_dev_consolidate(amr_dev *d, const amr_merge_job *jobs, int n)
 {
-   int rc = refine_data(d, jobs, n, false);
+   int rc = amr_merge_impl(d, jobs, n);
    if (!rc && n && d->tape && d->tape->on && !d->replaying) {
       const int first = (int) d->tape->merges.size();
       d->tape->merges.insert(d->tape->merges.end(), jobs, jobs + n);
@@ -1043,8 +1290,11 @@ int amr_dev_stage_fused(amr_dev *d, int start, int num, int stage, int permute, 
    // 1-7% slower fused; the 16^3, 40-variable bandwidth-scale run 15-18%
    // faster)
    const double cells = (double) d->n_active * num * d->g.nx * d->g.ny * d->g.nz;
-   if (!d->two_interiors || permute || d->whole_ghosts || (d->tape && d->tape->on) ||
-       d->replaying || (d->fused_mode == 1 && cells < 1.0e8))
+   // a 7-point stage that reads every face in place is one launch at any size,
+   // and the order of the phases does not matter to it
+   if (!d->two_interiors || !d->closed || (permute && !d->all_faces) || d->whole_ghosts ||
+       (d->tape && d->tape->on) || d->replaying ||
+       (d->fused_mode == 1 && cells < 1.0e8 && !d->all_faces))
       return amr_dev_stage(d, start, num, stage, permute, sum_row);
    if (start < 0 || num < 0 || start + num > d->c.num_vars)
       return amr_set_error(d, AMR_ERR_ARG, "stage: variables out of range");
@@ -1052,9 +1302,9 @@ int amr_dev_stage_fused(amr_dev *d, int start, int num, int stage, int permute, 
       return amr_set_error(d, AMR_ERR_ARG, "stage: checksum row %d not reserved", sum_row);
    if (!num)
       return AMR_OK;
-   if (!d->timing_dirs)
+   if (!d->timing_dirs && !d->all_faces)
       amr_span_begin(d, 0);
-   for (int dir = 0; dir < 3; dir++) {
+   for (int dir = 0; dir < 3 && !d->all_faces; dir++) {
       if (d->timing_dirs)
          amr_span_begin(d, kSpanExchangeX + dir);
       int rc = amr_launch_exchange_fused_dir(d, dir, start, num);
@@ -1063,7 +1313,7 @@ int amr_dev_stage_fused(amr_dev *d, int start, int num, int stage, int permute, 
       if (rc)
          return rc;
    }
-   if (!d->timing_dirs)
+   if (!d->timing_dirs && !d->all_faces)
       amr_span_end(d);
    amr_span_begin(d, 1);
    int rc = amr_launch_stencil_fused(d, start, num, sum_row >= 0);

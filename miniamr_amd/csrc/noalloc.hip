@@ -84,6 +84,8 @@ extern "C" int amr_dev_split_noalloc(amr_dev *d, const amr_split_job *jobs, int 
    if (!ptr)
       return amr_set_error(d, AMR_ERR_STATE, "split_noalloc: static scratch of device %d not "
                            "initialised", d->c.device);
+   if (int rc = amr_split_slots_current(d, jobs, n))
+      return rc;
    const int chunk = (int) std::min<size_t>((size_t) n, room / per_job);
    // earlier work of this context may still read a previous call's jobs
    HIP_TRY(d, hipStreamSynchronize(d->stream));

@@ -33,7 +33,7 @@ namespace {
 
 using namespace amrk;
 
-template <typename T, int ST, int NCOL, int NPER, int VPW, int NZ, int D = kDepth>
+template <typename T, int ST, int NCOL, int NPER, int VPW, int NZ>
 __global__ __launch_bounds__(kThreads) void k_stencil(T *__restrict__ pool,
                                                        const int32_t *__restrict__ sorted,
                                                        Lay L, int var0, int var_end,
@@ -52,7 +52,7 @@ __global__ __launch_bounds__(kThreads) void k_stencil(T *__restrict__ pool,
    const int v0 = var0 + vg * VPW;
    const int nv = min(VPW, var_end - v0);
    T *rec = pool + (int64_t) v0 * L.var_stride + (int64_t) sorted[in] * L.rec;
-   stencil_block<T, ST, NCOL, NPER, VPW, kThreads, NZ, D>(rec, L, nv, (A *) smem, red,
+   stencil_block<T, ST, NCOL, NPER, VPW, kThreads, NZ>(rec, L, nv, (A *) smem, red,
                                          partials ? partials + (int64_t) v0 * part_stride + in
                                                   : nullptr,
                                          part_stride);
@@ -217,16 +217,6 @@ static int xcd_remap_on()
    return v;
 }
 
-static int depth6()
-{
-   static int v = -1;
-   if (v < 0) {
-      const char *e = getenv("MINIAMR_STENCIL_DEPTH");
-      v = e && atoi(e) == 6;
-   }
-   return v;
-}
-
 // The vector form (k_stencil_v16) serves 27-point stencils of 16 x 16
 // faces whose interiors and x faces start on 16-byte boundaries, unless
 // MINIAMR_STENCIL_VEC=0.  Plain and fused stages then both use it, so their
@@ -248,6 +238,13 @@ static bool use_vec(const amr_dev *d, int st)
    const Lay &g = d->g;
    return st == 27 && g.ny == 16 && g.nz == 16 && stencil_vec_on() && d->oI_par[0] % C == 0 &&
           d->oI_par[1] % C == 0 && g.oF[0] % C == 0 && g.oF[1] % C == 0 && g.rec % C == 0;
+}
+
+bool uses_vec(const amr_dev *d)
+{
+   return d->c.precision == AMR_PREC_F64   ? use_vec<double>(d, d->g.stencil)
+          : d->c.precision == AMR_PREC_F32 ? use_vec<float>(d, d->g.stencil)
+                                           : use_vec<uint16_t>(d, d->g.stencil);
 }
 
 template <typename T, bool FUSED>
@@ -276,15 +273,9 @@ int launch_st_v(amr_dev *d, int start, int num, double *parts)
    hipLaunchKernelGGL((k_stencil<T, ST, NC, NP, V, NZ>), grid, dim3(kThreads), lds, d->stream, \
                       (T *) d->pool, d->d_sorted, L, start, start + num, parts,             \
                       d->c.max_blocks, xcd_remap_on())
-   // common face widths get a compile-time nz (constant LDS offsets)
+   // 16-cell rows get a compile-time nz (constant LDS offsets)
    if (ncol <= kThreads && plane <= 2 * kThreads) {
-      if (L.nz == 16 && depth6())
-         hipLaunchKernelGGL((k_stencil<T, ST, 1, 2, V, 16, 6>), grid, dim3(kThreads), lds,
-                            d->stream, (T *) d->pool, d->d_sorted, L, start, start + num, parts,
-                            d->c.max_blocks, xcd_remap_on());
-      else if (L.nz == 16) GO(1, 2, 16);
-      else if (L.nz == 12) GO(1, 2, 12);
-      else if (L.nz == 8) GO(1, 2, 8);
+      if (L.nz == 16) GO(1, 2, 16);
       else GO(1, 2, 0);
    } else if (ncol <= 2 * kThreads && plane <= 4 * kThreads)
       GO(2, 4, 0);
@@ -306,6 +297,12 @@ int launch_st(amr_dev *d, int start, int num, double *parts)
       if (int rc = amr_lay(d, start, num, &L))
          return rc;
       return launch_v16<T, false>(d, L, L, start, num, parts);
+   }
+   if (amr_box_fits(d, ST)) {   // the whole-box form, where the box fits in LDS
+      Lay L;
+      if (int rc = amr_lay(d, start, num, &L))
+         return rc;
+      return amr_launch_box(d, ST, nullptr, nullptr, L, L, start, num, parts);
    }
    if (stencil_vpw<T>() == 4)
       return launch_st_v<T, ST, 4>(d, start, num, parts);
@@ -341,8 +338,6 @@ int launch_fused_v(amr_dev *d, int start, int num, double *parts)
                       start + num, parts, d->c.max_blocks, xcd_remap_on())
    if (ncol <= kThreads && plane <= 2 * kThreads) {
       if (L.nz == 16) GO(1, 2, 16);
-      else if (L.nz == 12) GO(1, 2, 12);
-      else if (L.nz == 8) GO(1, 2, 8);
       else GO(1, 2, 0);
    } else if (ncol <= 2 * kThreads && plane <= 4 * kThreads)
       GO(2, 4, 0);
@@ -371,6 +366,17 @@ int launch_fused(amr_dev *d, int start, int num, double *parts)
          return rc;
       for (int v = start; v < start + num; v++)
          d->par[v] ^= 1;   // the variables' cells now live in the other copy
+      return AMR_OK;
+   }
+   if (amr_box_fits(d, ST)) {   // the whole-box form, where the box fits in LDS
+      Lay L;
+      if (int rc = amr_lay(d, start, num, &L))
+         return rc;
+      if (int rc = amr_launch_box(d, ST, d->d_faces, d->d_edges, L, amr_lay_other(d, L), start,
+                                  num, parts))
+         return rc;
+      for (int v = start; v < start + num; v++)
+         d->par[v] ^= 1;
       return AMR_OK;
    }
    if (stencil_vpw<T>() == 4)
@@ -414,6 +420,12 @@ int launch_convert(amr_dev *d, int slot, bool in)
 }
 
 }  // namespace
+
+bool amr_uses_box(const amr_dev *d)
+{
+   return (d->g.stencil == 7 || d->g.stencil == 27) && !uses_vec(d) &&
+          amr_box_fits(d, d->g.stencil);
+}
 
 int amr_launch_stencil_fused(amr_dev *d, int start, int num, bool want_partials)
 {
