@@ -238,7 +238,12 @@ struct amr_dev {
    // slot was last written or active ([slot][variable]; two interiors only).
    std::vector<uint8_t> slot_par;
    std::vector<uint8_t> active;     // per slot: in the active list (two interiors only)
+   bool group_lds_set = false;      // k_mat_group's LDS limit raised
 };
+
+// amr_dev::d_check_counts: kCountSlots pairs of counters, kCountStride values
+// (a 128-byte line) apart; their sum is the count.
+constexpr int kCountSlots = 64, kCountStride = 16;
 
 // Storage helpers: T is double, float or uint16_t (bfloat16 bits); A is the
 // accumulation type (double for FP64 storage, float otherwise).
@@ -477,6 +482,11 @@ void amr_slot_written(amr_dev *d, int slot);
 int amr_launch_exchange_dir(amr_dev *d, int dir, int start, int num);
 int amr_launch_exchange_fused_dir(amr_dev *d, int dir, int start, int num);
 int amr_launch_stencil(amr_dev *d, int start, int num, bool want_partials, int calc_stage);
+// All groups of material variables of a --stencil 0 stage in one launch
+// (variable 0, and in calculation stages 0-3 variable 1, done before), where
+// a group's boxes fit in LDS.
+bool amr_mat_groups_fit(const amr_dev *d);
+int amr_launch_mat_groups(amr_dev *d, int calc_stage);
 // The whole-box stencil (box.hip; st: 7 or 27) where the block's ghost box fits
 // in LDS: interiors read in copy L and written in copy Lo, face ghosts where
 // faces says (null: the block's own ghost planes), 27-point edges where edges

@@ -134,8 +134,9 @@ int amr_dev_create(const amr_dev_config *cfg, amr_dev **out)
    d->h_pinned_bytes = sizeof(double) * std::max<size_t>(4096, (size_t) cfg->num_vars * 64);
    HIP_TRY(d, hipHostMalloc((void **) &d->h_pinned, d->h_pinned_bytes, hipHostMallocDefault));
    if (cfg->stencil == 0) {
-      HIP_TRY(d, hipMalloc(&d->d_check_counts, 2 * sizeof(unsigned long long)));
-      HIP_TRY(d, hipMemsetAsync(d->d_check_counts, 0, 2 * sizeof(unsigned long long), d->stream));
+      const size_t bytes = sizeof(unsigned long long) * kCountSlots * kCountStride;
+      HIP_TRY(d, hipMalloc(&d->d_check_counts, bytes));
+      HIP_TRY(d, hipMemsetAsync(d->d_check_counts, 0, bytes, d->stream));
    }
    HIP_TRY(d, hipStreamSynchronize(d->stream));
    return AMR_OK;
@@ -994,11 +995,12 @@ int amr_dev_read_check_counts(amr_dev *d, int64_t counts[2])
    counts[0] = counts[1] = 0;
    if (!d->d_check_counts)
       return AMR_OK;
-   unsigned long long h[2];
+   unsigned long long h[kCountSlots * kCountStride];
    HIP_TRY(d, hipStreamSynchronize(d->stream));
    HIP_TRY(d, hipMemcpy(h, d->d_check_counts, sizeof(h), hipMemcpyDeviceToHost));
-   counts[0] = (int64_t) h[0];
-   counts[1] = (int64_t) h[1];
+   for (int t = 0; t < kCountSlots; t++)
+      for (int i = 0; i < 2; i++)
+         counts[i] += (int64_t) h[t * kCountStride + i];
    return AMR_OK;
 }
 

@@ -36,7 +36,7 @@ struct MatArgs {
    int var, mat;
    double a1;
    const double *a0;          // mat values (device)
-   unsigned long long *counts;  // [0] clamps that divide, [1] that scale
+   unsigned long long *counts;  // slot pairs: [0] clamps that divide, [1] that scale
 };
 
 // One block's cells of every variable.
@@ -87,6 +87,9 @@ __device__ __forceinline__ A clamp(A v, const MatArgs &m, unsigned &ndiv, unsign
    return v;
 }
 
+// The clamps of a wavefront, added to one of kCountSlots counter pairs, each on
+// a line of its own: with one pair for all, the whole-stage launch (7,000
+// wavefronts) spent 150 of its 200 us on those two addresses.
 __device__ __forceinline__ void add_counts(const MatArgs &m, unsigned ndiv, unsigned nmul)
 {
    for (int o = 32; o > 0; o >>= 1) {
@@ -94,8 +97,11 @@ __device__ __forceinline__ void add_counts(const MatArgs &m, unsigned ndiv, unsi
       nmul += __shfl_down(nmul, o, 64);
    }
    if ((threadIdx.x & 63) == 0 && (ndiv | nmul)) {
-      atomicAdd(&m.counts[0], (unsigned long long) ndiv);
-      atomicAdd(&m.counts[1], (unsigned long long) nmul);
+      unsigned long long *const c =
+         m.counts + ((blockIdx.x + 5 * blockIdx.y + 11 * (threadIdx.x >> 6)) & (kCountSlots - 1)) *
+                       kCountStride;
+      atomicAdd(&c[0], (unsigned long long) ndiv);
+      atomicAdd(&c[1], (unsigned long long) nmul);
    }
 }
 
@@ -259,6 +265,193 @@ __global__ __launch_bounds__(kThreads) void k_mat_commit(T *pool, const int32_t 
    add_counts(m, ndiv, nmul);
 }
 
+// ---- a whole stage
+// The variables (u, mat+u, 2*mat+u, 3*mat+u) form a group: apart from
+// variables 0 and 1, an update reads no variable outside its group.  So once
+// variable 0 and, in calculation stages 0-3, variable 1 are done, the groups
+// are independent: one launch, one workgroup per (block, group), the four
+// variables in class order.  One launch per variable left the device with one
+// workgroup per block at a time (176 blocks: 19 x 59 us for stage 5).  The
+// group's boxes stay in LDS throughout: each cell is read once and written
+// once, and no neighbour read computes a record offset.
+constexpr int kGroupThreads = 512;
+constexpr size_t kGroupLds = 156 * 1024;
+
+template <typename T>
+size_t group_lds(const Lay &L)
+{
+   return sizeof(typename Acc<T>::type) *
+          (4 * (size_t) L.gx * L.gy * L.gz + (size_t) L.nx * L.ny * L.nz);
+}
+
+template <typename T>
+__global__ __launch_bounds__(kGroupThreads) void k_mat_group(T *pool, const int32_t *sorted,
+                                                             Lay L, MatArgs m, int op)
+{
+   typedef typename Acc<T>::type A;
+   extern __shared__ __align__(16) unsigned char smem[];
+   const int u = blockIdx.y, mat = m.mat;
+   const int nbox = L.gx * L.gy * L.gz, ncell = L.nx * L.ny * L.nz, sy = L.gz, sx = L.gy * L.gz;
+   A *const box = (A *) smem, *const tmp = box + 4 * nbox;
+   T *const rec = pool + (int64_t) sorted[blockIdx.x] * L.rec;
+   const T *const i0 = rec + L.oI, *const i1 = rec + L.var_stride + L.oI;   // variables 0 and 1
+   const A a1 = A(m.a1), one = A(1.0);
+   const int first = op < 4 ? 2 : 1;   // variables below are done
+   const int tid = threadIdx.x;
+   auto stored = [](A v) { return to_acc(from_acc<T>(v)); };
+   unsigned ndiv = 0, nmul = 0;
+   // cell t of the record's order of variable var (and its z-plane copy)
+   auto put = [&](int var, int t, A v) {
+      const int i = t / (L.ny * L.nz), r = t - i * L.ny * L.nz, j = r / L.nz, k = r - j * L.nz;
+      T *const out = rec + (int64_t) var * L.var_stride;
+      const T x = from_acc<T>(v);
+      out[L.oI + t] = x;
+      if (k == 0) out[L.oZI + i * L.ny + j] = x;
+      if (k == L.nz - 1) out[L.oZI + (L.nx + i) * L.ny + j] = x;
+   };
+   if (op <= 3) {
+      // pointwise updates: class 0, and in stage 0 all classes, which read
+      // each other at one cell only -- no box needed
+      for (int t = tid; t < ncell; t += kGroupThreads) {
+         const A p0 = to_acc(i0[t]), p1 = to_acc(i1[t]);
+         A v[4];
+#pragma unroll
+         for (int c = 0; c < 4; c++)
+            if (c == 0 || op == 0)
+               v[c] = to_acc(rec[(int64_t) (c * mat + u) * L.var_stride + L.oI + t]);
+         if (u >= first) {
+            A r;
+            if (op != 0) r = v[0] + v[0] * ((p0 + p1) - a1 * v[0]) / (A(m.a0[u]) + p1);
+            else r = v[0] + v[0] * ((p0 + p1) - a1 * v[0]);
+            put(u, t, clamp(r, m, ndiv, nmul));
+         }
+         if (op != 0)
+            continue;
+         if (mat + u >= first) {
+            v[1] = v[1] * (((p0 + v[1]) + a1 * v[2]) + (one - a1) * v[3]) / p1;
+            v[1] = stored(clamp(v[1], m, ndiv, nmul));
+            put(mat + u, t, v[1]);
+         }
+         const A a0 = A(m.a0[u]);
+         v[2] = v[2] + v[1] * ((a1 * p0 + a0 * v[2]) + (one - a1) * v[3]) / p1;
+         v[2] = stored(clamp(v[2], m, ndiv, nmul));
+         put(2 * mat + u, t, v[2]);
+         v[3] = v[3] + v[1] * (((a1 * p0 + a0 * v[3]) + (one - a0) * v[2]) + (one - a1) * v[1]) /
+                          (p1 * p1);
+         put(3 * mat + u, t, clamp(v[3], m, ndiv, nmul));
+      }
+      if (op == 0) {
+         add_counts(m, ndiv, nmul);
+         return;
+      }
+   }
+   // boxes of classes lo..3
+   const int lo = op <= 3 ? 1 : 0;
+   for (int e = tid; e < nbox; e += kGroupThreads) {
+      const int i = e / sx, r = e - i * sx, j = r / sy, k = r - j * sy, h = home(L, i, j, k);
+#pragma unroll
+      for (int c = 0; c < 4; c++)
+         if (c >= lo)
+            box[(c - lo) * nbox + e] = to_acc(rec[(int64_t) (c * mat + u) * L.var_stride + h]);
+   }
+   __syncthreads();
+   // LDS place of interior cell t of the record's order
+   auto at = [&](int t) {
+      const int i = t / (L.ny * L.nz), r = t - i * L.ny * L.nz, j = r / L.nz, k = r - j * L.nz;
+      return (i + 1) * sx + (j + 1) * sy + k + 1;
+   };
+   const A *const c1 = box + (1 - lo) * nbox, *const c2 = c1 + nbox, *const c3 = c2 + nbox;
+   for (int cls = lo; cls < 4; cls++) {
+      const int var = cls * mat + u;
+      if (var < first)
+         continue;
+      A *const me = box + (cls - lo) * nbox;
+      if (op <= 3) {
+         // in-place sweep, a thread per line (k_mat_sweep's expressions)
+         const int ax = op - 1;
+         const int n = ax == 0 ? L.nx : ax == 1 ? L.ny : L.nz;
+         const int n1 = ax == 0 ? L.ny : L.nx, n2 = ax == 2 ? L.ny : L.nz;
+         const int s = ax == 0 ? sx : ax == 1 ? sy : 1;
+         const int s1 = ax == 0 ? sy : sx, s2 = ax == 2 ? sy : 1;
+         const int r0 = ax == 0 ? L.ny * L.nz : ax == 1 ? L.nz : 1;   // step in record order
+         const int r1 = ax == 0 ? L.nz : L.ny * L.nz, r2 = ax == 2 ? L.nz : 1;
+         const A a0 = A(m.a0[u]);
+         for (int t = tid; t < n1 * n2; t += kGroupThreads) {
+            const int l1 = t / n2, l2 = t - l1 * n2;
+            const int b0 = (l1 + 1) * s1 + (l2 + 1) * s2, g0 = l1 * r1 + l2 * r2;
+            A prev = me[b0];
+            for (int p = 1; p <= n; p++) {
+               const int q = b0 + p * s, g = g0 + (p - 1) * r0;
+               const A v = me[q], vn = me[q + s], q1 = to_acc(i1[g]);
+               const A gv = cls == 1 ? v : c1[q];
+               const A gm = cls == 1 ? prev : c1[q - s];
+               const A gp = cls == 1 ? vn : c1[q + s];
+               const A tmp1 = fabs(gv - gm), tmp2 = fabs(gv - gp);
+               const A w = tmp1 > tmp2 ? tmp1 - tmp2 : tmp2 - tmp1;
+               const A num = ((tmp1 * prev) + (w * (v + q1))) + (tmp2 * vn);
+               A den;
+               if (cls == 1) {
+                  den = ((((a1 + a0) + prev) + v) + vn) + to_acc(i0[g]);
+                  den = den + q1;
+               } else {
+                  den = cls == 2 ? ((a1 + a0) + c1[q]) + c3[q] : ((a1 + a0) + c2[q]) + c1[q];
+                  den = ((den + prev) + v) + vn;
+               }
+               prev = stored(num / den);
+               me[q] = prev;
+            }
+         }
+         __syncthreads();
+         for (int t = tid; t < ncell; t += kGroupThreads) {
+            const int q = at(t);
+            me[q] = stored(clamp(me[q], m, ndiv, nmul));
+         }
+      } else {
+         const A *const qx = box + (cls + kPartner[cls][0]) * nbox,
+                 *const qy = box + (cls + kPartner[cls][1]) * nbox,
+                 *const qz = box + (cls + kPartner[cls][2]) * nbox;
+         for (int t = tid; t < ncell; t += kGroupThreads) {
+            const int q = at(t);
+            const A v = me[q];
+            A r;
+            if (op == 4) {
+               A s = me[q - sx] * qx[q - sx];
+               s = s + me[q - sy] * qy[q - sy];
+               s = s + me[q - 1] * qz[q - 1];
+               s = s + v * v;
+               s = s + me[q + 1] * qz[q + 1];
+               s = s + me[q + sy] * qy[q + sy];
+               s = s + me[q + sx] * qx[q + sx];
+               r = s / A(7.0) * (a1 + v);
+            } else {
+               A s = A(0);
+#pragma unroll
+               for (int d = 0; d < 27; d++) {
+                  const int di = d / 9 - 1, dj = (d / 3) % 3 - 1, dk = d % 3 - 1;
+                  const int nz = (di != 0) + (dj != 0) + (dk != 0);   // non-zero offsets
+                  const A *const src = nz == 0 ? me : nz == 1 ? qx : nz == 2 ? qy : qz;
+                  const A e = src[q + di * sx + dj * sy + dk];
+                  s = d ? s + e : e;
+               }
+               r = s / (a1 + A(27.0));
+            }
+            tmp[t] = r;
+         }
+         __syncthreads();
+         for (int t = tid; t < ncell; t += kGroupThreads)
+            me[at(t)] = stored(clamp(tmp[t], m, ndiv, nmul));
+      }
+      __syncthreads();
+   }
+   for (int t = tid; t < ncell; t += kGroupThreads) {
+      const int q = at(t);
+      for (int cls = lo; cls < 4; cls++)
+         if (cls * mat + u >= first)
+            put(cls * mat + u, t, box[(cls - lo) * nbox + q]);
+   }
+   add_counts(m, ndiv, nmul);
+}
+
 template <typename T>
 int launch_mat(amr_dev *d, int var, int calc_stage)
 {
@@ -299,7 +492,56 @@ int launch_mat(amr_dev *d, int var, int calc_stage)
    return AMR_OK;
 }
 
+template <typename T>
+int launch_group(amr_dev *d, int calc_stage)
+{
+   Lay L;
+   if (int rc = amr_lay(d, 0, d->c.num_vars, &L))
+      return rc;
+   MatArgs m;
+   m.var = 0;
+   m.mat = d->mat;
+   m.a1 = d->a1;
+   m.a0 = d->d_a0;
+   m.counts = d->d_check_counts;
+   // stage 0 needs no box, the sweeps those of classes 1-3 (two workgroups
+   // per CU at 12^3 FP64), the Jacobi updates four and the new values
+   const int op = calc_stage % 6;
+   const size_t lds = op == 0 ? 0
+                    : op <= 3 ? sizeof(typename Acc<T>::type) * 3 * (size_t) L.gx * L.gy * L.gz
+                              : group_lds<T>(L);
+   if (!d->group_lds_set) {   // more than the default limit of a launch
+      HIP_TRY(d, hipFuncSetAttribute((const void *) &k_mat_group<T>,
+                                     hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     (int) kGroupLds));
+      d->group_lds_set = true;
+   }
+   hipLaunchKernelGGL(k_mat_group<T>, dim3(d->n_active, d->mat), dim3(kGroupThreads), lds,
+                      d->stream, (T *) d->pool, d->d_sorted, L, m, op);
+   HIP_TRY(d, hipGetLastError());
+   return AMR_OK;
+}
+
 }  // namespace
+
+bool amr_mat_groups_fit(const amr_dev *d)
+{
+   return (d->c.precision == AMR_PREC_F64 ? group_lds<double>(d->g) : group_lds<float>(d->g)) <=
+          kGroupLds;
+}
+
+int amr_launch_mat_groups(amr_dev *d, int calc_stage)
+{
+   if (!d->n_active)
+      return AMR_OK;
+   if (!d->d_a0)
+      return amr_set_error(d, AMR_ERR_STATE, "stencil 0: amr_dev_set_materials not called");
+   switch (d->c.precision) {
+   case AMR_PREC_F64: return launch_group<double>(d, calc_stage);
+   case AMR_PREC_F32: return launch_group<float>(d, calc_stage);
+   default: return launch_group<uint16_t>(d, calc_stage);
+   }
+}
 
 // One variable's update of a --stencil 0 stage other than the plain 7-point
 // ones (variable 0 and variables >= 4*mat are left to the caller).

@@ -451,12 +451,36 @@ int amr_launch_stencil_fused(amr_dev *d, int start, int num, bool want_partials)
 // variables from 4*mat on take the 7-point average, the others the
 // variable-work updates.  Checksum partials come from a block-sum pass.
 template <typename T>
+int launch_average0(amr_dev *d, int start, int num)   // the 7-point average
+{
+   if (!amr_box_fits(d, 7))
+      return launch_st_v<T, 7, 1>(d, start, num, nullptr);
+   Lay L;
+   if (int rc = amr_lay(d, start, num, &L))
+      return rc;
+   return amr_launch_box(d, 7, nullptr, nullptr, L, L, start, num, nullptr);
+}
+
+template <typename T>
 int launch_stencil0(amr_dev *d, int start, int num, bool want_partials, int calc_stage)
 {
    if (!d->n_active || !num)
       return AMR_OK;
+   if (start == 0 && num == d->c.num_vars && amr_mat_groups_fit(d)) {
+      // a whole stage: the same updates by groups of variables
+      int rc = launch_average0<T>(d, 0, 1);
+      if (!rc && calc_stage % 6 < 4)
+         rc = amr_launch_mat_stencil(d, 1, calc_stage);
+      if (!rc)
+         rc = amr_launch_mat_groups(d, calc_stage);
+      if (!rc && num > 4 * d->mat)
+         rc = launch_average0<T>(d, 4 * d->mat, num - 4 * d->mat);
+      if (rc)
+         return rc;
+      return want_partials ? launch_block_sums<T>(d, start, num) : AMR_OK;
+   }
    for (int v = start; v < start + num; v++) {
-      int rc = (v == 0 || v >= 4 * d->mat) ? launch_st_v<T, 7, 1>(d, v, 1, nullptr)
+      int rc = (v == 0 || v >= 4 * d->mat) ? launch_average0<T>(d, v, 1)
                                            : amr_launch_mat_stencil(d, v, calc_stage);
       if (rc)
          return rc;
