@@ -516,4 +516,4 @@ int amr_launch_split(amr_dev *d, const amr_split_job *d_jobs, int n, void *scrat
 int amr_noalloc_init(amr_dev *d);
 int amr_launch_merge(amr_dev *d, const amr_merge_job *d_jobs, int n, void *scratch);
 int amr_launch_convert_in(amr_dev *d, int slot);
-int amr_launch_convert_out(amr_dev *d, int slot);
+int amr_launch_convert_out(amr_dev *d, int slot, double *out);   // out: device address

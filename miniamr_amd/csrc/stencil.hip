@@ -402,19 +402,19 @@ int launch_block_sums(amr_dev *d, int start, int num)
 }
 
 template <typename T>
-int launch_convert(amr_dev *d, int slot, bool in)
+int launch_convert(amr_dev *d, int slot, double *out)   // out null: d_stage to the record
 {
    int cells = d->g.gx * d->g.gy * d->g.gz;
    dim3 grid((cells + 255) / 256, d->c.num_vars);
    Lay L;
    if (int rc = amr_lay(d, 0, d->c.num_vars, &L))
       return rc;
-   if (in)
+   if (!out)
       hipLaunchKernelGGL(k_convert_in<T>, grid, dim3(256), 0, d->stream, (T *) d->pool,
                          (const double *) d->d_stage, L, slot, cells);
    else
       hipLaunchKernelGGL(k_convert_out<T>, grid, dim3(256), 0, d->stream,
-                         (const T *) d->pool, d->d_stage, L, slot, cells);
+                         (const T *) d->pool, out, L, slot, cells);
    HIP_TRY(d, hipGetLastError());
    return AMR_OK;
 }
@@ -532,17 +532,17 @@ int amr_launch_reduce_sums(amr_dev *d, int start, int num, double *dst_row)
 int amr_launch_convert_in(amr_dev *d, int slot)
 {
    switch (d->c.precision) {
-   case AMR_PREC_F64: return launch_convert<double>(d, slot, true);
-   case AMR_PREC_F32: return launch_convert<float>(d, slot, true);
-   default: return launch_convert<uint16_t>(d, slot, true);
+   case AMR_PREC_F64: return launch_convert<double>(d, slot, nullptr);
+   case AMR_PREC_F32: return launch_convert<float>(d, slot, nullptr);
+   default: return launch_convert<uint16_t>(d, slot, nullptr);
    }
 }
 
-int amr_launch_convert_out(amr_dev *d, int slot)
+int amr_launch_convert_out(amr_dev *d, int slot, double *out)
 {
    switch (d->c.precision) {
-   case AMR_PREC_F64: return launch_convert<double>(d, slot, false);
-   case AMR_PREC_F32: return launch_convert<float>(d, slot, false);
-   default: return launch_convert<uint16_t>(d, slot, false);
+   case AMR_PREC_F64: return launch_convert<double>(d, slot, out);
+   case AMR_PREC_F32: return launch_convert<float>(d, slot, out);
+   default: return launch_convert<uint16_t>(d, slot, out);
    }
 }

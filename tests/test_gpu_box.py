@@ -110,3 +110,32 @@ def test_inactive_slots_and_saved_states():
     for s in range(24):
         assert np.array_equal(fresh.download(s), want[s]), s
         assert np.array_equal(g.download(s), want[s]), s
+
+
+@pytest.mark.parametrize("prec", [M.PREC_F64, M.PREC_F32, M.PREC_BF16], ids=["f64", "f32", "bf16"])
+def test_download_into_page_locked_memory(prec):
+    """A download into page-locked memory (written by the conversion kernel
+    itself) gives the values of one into pageable memory, at the start, in the
+    middle and at the end of the allocation, and leaves its neighbours alone."""
+    require(M.LIB_PATH, "run __graft_entry__.build()")
+    import ctypes
+    lib = M.load_library(M.LIB_PATH)
+    hip = ctypes.CDLL("libamdhip64.so")
+    d = M.Device(nx=6, ny=4, nz=10, num_vars=3, max_blocks=2, stencil=7, precision=prec, lib=lib)
+    rng = np.random.default_rng(2)
+    d.upload(1, rng.random(d.shape))
+    want = d.download(1)
+    n, lead = want.size, 5
+    ptr = ctypes.c_void_p()
+    assert hip.hipHostMalloc(ctypes.byref(ptr), ctypes.c_size_t(8 * (3 * n + lead)), 0) == 0
+    buf = np.ctypeslib.as_array((ctypes.c_double * (3 * n + lead)).from_address(ptr.value))
+    try:
+        for at in (0, lead, n + lead, 2 * n + lead):
+            buf[:] = -1.0
+            out = ctypes.cast(ptr.value + 8 * at, ctypes.POINTER(ctypes.c_double))
+            assert lib.amr_dev_download_block(d.h, 1, out) == 0
+            assert np.array_equal(buf[at:at + n], want.ravel())
+            assert np.all(buf[:at] == -1.0) and np.all(buf[at + n:] == -1.0)
+    finally:
+        d.close()
+        hip.hipHostFree(ptr)
