@@ -258,23 +258,24 @@ int amr_dev_stage(amr_dev *dev, int start, int num, int stage, int permute,
  * last one of a timestep that ends in a refinement or ends the run).
  * Cells, checksums and every ghost value a stencil reads are those of
  * amr_dev_stage.  The difference is where they come from: the ghost planes
- * of same-level faces of blocks away from the domain boundary, and their
- * 27-point edge extensions, are not written -- the stencil reads those
- * cells from the neighbours' interiors, which stay unchanged because the
- * stage writes its results to a second copy of every interior (records
- * hold two unless the context was created with MINIAMR_FUSED=0 in the
- * environment, which costs ~70% more pool memory at 16^3).  Those ghost
- * cells are stale until the next amr_dev_stage or amr_dev_comm of the same
- * variables; set_mesh, split, consolidate, stencil, download_block, the
- * halo codec and save_state first bring them up to date (to the values
- * amr_dev_stage would have written, from the interiors the stage read).
+ * of same-level and boundary faces, and the 27-point edges, are not
+ * written -- the stencil reads those cells from the neighbours' (or the
+ * block's own) interiors, which stay unchanged because the stage writes its
+ * results to a second copy of every interior (records hold two unless the
+ * context was created with MINIAMR_FUSED=0 in the environment, which costs
+ * ~70% more pool memory at 16^3).  Those ghost cells are stale until the
+ * next amr_dev_stage or amr_dev_comm of the same variables; set_mesh, split,
+ * consolidate, stencil, download_block, the halo codec and save_state first
+ * bring them up to date (to the values amr_dev_stage would have written,
+ * from the interiors the stage read).
  * With the 7-point stencil every ghost plane -- boundary and coarse/fine ones
  * too -- is read from where its values come from, at any stage size and
  * with permute, where the block's ghost box fits in LDS.  It is
  * amr_dev_stage without two interiors, with permute != 0, while the tape
- * records, when the jobs name blocks outside the active list, and for
- * stages of fewer than 1e8 cell updates (latency-bound; MINIAMR_FUSED=2 at
- * creation fuses those too). */
+ * records, when the jobs name blocks outside the active list, and -- where
+ * edges are not folded (MINIAMR_FOLD_EDGES=0, a coarse/fine plane with
+ * quarters missing, 7-point boxes too large for LDS) -- for stages of fewer
+ * than 1e8 cell updates (MINIAMR_FUSED=2 at creation fuses those too). */
 int amr_dev_stage_fused(amr_dev *dev, int start, int num, int stage, int permute,
                         int sum_row);
 

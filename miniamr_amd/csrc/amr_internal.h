@@ -59,8 +59,14 @@ struct FusedJob {
    amr_face_job jb;
    int32_t mode;
    int32_t alt[4];
-   int32_t pad;
+   // coarse/fine jobs, edges folded: the block's boundary faces of earlier
+   // directions (bit f: face f).  In the plain stage their fills have copied
+   // this plane's ghost cells next to them, as the previous stage left them,
+   // to the ring; the job does so before it writes the new values.
+   int32_t ring;
 };
+// An in-place face (redir) that is the domain boundary: the block's own plane.
+enum { kRedirBc = -2 };
 
 // Where a fused stage finds the cells of one ghost edge line or corner of a
 // block: kEdgeSrcs entries per slot, in this order
@@ -188,13 +194,13 @@ struct amr_dev {
    // The plan of amr_dev_stage_fused, derived from the plain plan by
    // set_mesh: reduced job lists per direction, and per active block
    // (sorted order) the slots its six faces are read from in place (-1:
-   // its own ghost plane).  stale[v]: variable v's in-place faces' ghost
+   // its own ghost plane; kRedirBc: its own plane next to the boundary).  stale[v]: variable v's in-place faces' ghost
    // planes have not been written since the last plain exchange.
    FusedJob *d_fjobs = nullptr;
    int32_t fcount[3] = {0, 0, 0};
    int fjobs_cap = 0;
-   // the plain jobs of the faces a fused stage reads in place (same-level
-   // jobs of blocks without a boundary face), per direction: rerun on the
+   // edges not folded: the plain jobs of the faces a fused stage reads in place
+   // (same-level jobs of blocks without a boundary face), per direction: rerun on the
    // interiors the last fused stage read, they write the ghost cells that
    // stage left unwritten (amr_require_fresh)
    amr_face_job *d_mjobs = nullptr;

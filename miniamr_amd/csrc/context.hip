@@ -433,58 +433,79 @@ static bool fold_edges_on()
 }
 
 // Edge sources of a fused stage (EdgeSrc).  In the reference a ghost edge
-// cell of a block gets its value from the last job that writes it in a
-// stage (27-point stencil, --code 0; ref/comm.c:1597-1688): a cell with a z
-// ghost coordinate from the block's z-face job, which copies the z-plane
-// ring of its source; a cell with x and y ghost coordinates (z interior)
-// from the y-face job, which copies the source's x-extended rows; each
-// copies the source's cell at the same in-plane coordinates on the plane
-// next to the shared face.  Only same-level jobs of blocks without a
-// boundary face extend and are folded (a boundary block's jobs all run);
-// a prolongation or restriction writes no edge cell, which then keeps what
-// the slot held (stale).  Following these copies, and the in-place face
-// reads of the plan, back to a cell that some job in the stage does write
-// or that is an interior cell gives the value the stage's stencil sees.
+// cell of a block gets its value from the last fill that writes it in a
+// stage (27-point stencil, --code 0; ref/comm.c:1597-1688, 1911-1965): a
+// same-level y fill copies its source's x-extended rows, a same-level z fill
+// the whole ring of its source's z plane, a boundary fill the block's own
+// whole plane next to the face; a prolongation or restriction writes no edge
+// cell, which then keeps what the slot held (stale).  Following these copies
+// back to a cell that is an interior cell, a coarse/fine ghost cell or a
+// stale one gives the value the stage's stencil sees.
 namespace {
 
 struct Cell { int slot, i, j, k; };
 
+// How a face's ghost plane is filled, when not from a same-level block:
+// no job or a coarse/fine one (neither writes ring cells), or the boundary.
+enum { FK_NONE = -1, FK_BC = -2, FK_CF = -3 };
+
 struct EdgeResolver {
    const Lay &g;
-   const std::vector<int32_t> &same;
-   const std::vector<uint8_t> &bc;
+   const std::vector<int32_t> &kind;   // per slot and face: FK_*, or the same-level source
    Lay L0;   // g with the interior copies at offset 0 (ES_I / ES_ZI offsets)
 
-   EdgeResolver(const Lay &g_, const std::vector<int32_t> &same_, const std::vector<uint8_t> &bc_)
-      : g(g_), same(same_), bc(bc_), L0(g_)
+   EdgeResolver(const Lay &g_, const std::vector<int32_t> &kind_) : g(g_), kind(kind_), L0(g_)
    {
       L0.oI = 0;
       L0.oZI = 0;
    }
 
-   // the cell whose value block b's cell (i, j, k) holds when the stencil runs
+   // The cell whose value block b's cell (i, j, k) holds when the stencil
+   // runs: follow the last fill that wrote it, then the fill that had written
+   // the cell this one read by then (phases x, y, z: `p` is the last phase
+   // that counts), and so on.  A cell that no fill of those phases writes
+   // holds what the slot held before, except a coarse/fine ghost cell that a
+   // boundary fill of an earlier phase read: that is the previous stage's
+   // value, which the coarse/fine job copies to the cell of the boundary's
+   // edge line before it writes the new one (FusedJob::ring) -- so the chain
+   // ends at that edge cell.
    Cell resolve(int b, int i, int j, int k) const
    {
-      for (int hop = 0; hop < 8; hop++) {
-         const bool gi = i == 0 || i == g.nx + 1, gj = j == 0 || j == g.ny + 1,
-                    gk = k == 0 || k == g.nz + 1;
-         const int ng = gi + gj + gk;
-         if (!ng || bc[b])
+      int p = 2;
+      Cell last{b, i, j, k};
+      for (int hop = 0; hop < 12; hop++) {
+         const bool g3[3] = {i == 0 || i == g.nx + 1, j == 0 || j == g.ny + 1,
+                             k == 0 || k == g.nz + 1};
+         const int ng = g3[0] + g3[1] + g3[2];
+         if (!ng)
             return {b, i, j, k};
-         int f, src;
-         if (ng == 1)           // face interior: read in place, or the job writes it
-            f = gi ? (i != 0) : gj ? 2 + (j != 0) : 4 + (k != 0);
-         else if (gk)           // z ring: the z-face job's extension
-            f = 4 + (k != 0);
-         else                   // x and y ghost, z interior: the y-face job's extension
-            f = 2 + (j != 0);
-         src = same[6 * (size_t) b + f];
-         if (src < 0)
-            return {b, i, j, k};
-         b = src;
-         if (f < 2) i = (f & 1) ? 1 : g.nx;
-         else if (f < 4) j = (f & 1) ? 1 : g.ny;
-         else k = (f & 1) ? 1 : g.nz;
+         int d = p, src = FK_NONE;
+         for (; d >= 0; d--) {
+            if (!g3[d])
+               continue;
+            const int f = d == 0 ? (i != 0) : d == 1 ? 2 + (j != 0) : 4 + (k != 0);
+            src = kind[6 * (size_t) b + f];
+            // a same-level fill covers the ghosts of earlier directions only
+            const bool later = (d < 1 && g3[1]) || (d < 2 && g3[2]);
+            if (src == FK_BC || (src >= 0 && !later))
+               break;
+         }
+         if (d < 0) {
+            const int e = g3[0] ? 0 : g3[1] ? 1 : 2;
+            const int f = 2 * e + (e == 0 ? i != 0 : e == 1 ? j != 0 : k != 0);
+            return ng == 1 && e > p && kind[6 * (size_t) b + f] == FK_CF ? last : Cell{b, i, j, k};
+         }
+         last = {b, i, j, k};
+         const bool hi = d == 0 ? i != 0 : d == 1 ? j != 0 : k != 0;
+         const int n = d == 0 ? g.nx : d == 1 ? g.ny : g.nz;
+         int &c = d == 0 ? i : d == 1 ? j : k;
+         if (src == FK_BC) {
+            c = hi ? n : 1;
+         } else {
+            b = src;
+            c = hi ? 1 : n;
+         }
+         p = d - 1;
       }
       return {-1, 0, 0, 0};
    }
@@ -510,29 +531,26 @@ struct EdgeResolver {
       return true;
    }
 
-   // entry of a line of n cells, cell(t) giving block b's cell t (resolved
-   // when folding, else the block's own); false if the cells are not one
-   // affine run of one block and kind.  Every cell of a line follows the
-   // same copies (the jobs that write a line, and the in-place faces on the
-   // way, are those of its whole face), so the first two cells give the
-   // run and the last one checks it.
-   template <typename F>
-   bool line(int b, int axis, int n, F cell, bool fold, EdgeSrc &e) const
+   // entry of a line of n cells along `axis` from block b's cell c; false if
+   // they are not one affine run.  No copy on the way changes the coordinate
+   // along the line, and every cell of the line follows the same fills, so the
+   // first cell's source gives the others'.
+   bool line(const Cell &c, int axis, int n, bool fold, EdgeSrc &e) const
    {
-      auto at = [&](int t, EdgeSrc &x) {
-         const Cell c = cell(t);
-         return entry(fold ? resolve(b, c.i, c.j, c.k) : c, axis, x);
-      };
-      if (!at(0, e))
+      const Cell c0 = fold ? resolve(c.slot, c.i, c.j, c.k) : c;
+      if (!entry(c0, axis, e))
          return false;
+      auto at = [&](int t) {
+         Cell x = c0;
+         (axis == 0 ? x.i : axis == 1 ? x.j : x.k) += t;
+         EdgeSrc y;
+         entry(x, axis, y);
+         return y;
+      };
       if (n > 1) {
-         EdgeSrc e1, el;
-         if (!at(1, e1) || e1.slot != e.slot || e1.kind != e.kind)
-            return false;
+         const EdgeSrc e1 = at(1), el = at(n - 1);
          e.stride = e1.off - e.off;
-         if (n > 2 && (!at(n - 1, el) || el.slot != e.slot || el.kind != e.kind ||
-                       el.off != e.off + (n - 1) * e.stride))
-            return false;
+         return e1.kind == e.kind && el.kind == e.kind && el.off == e.off + (n - 1) * e.stride;
       }
       return true;
    }
@@ -544,21 +562,17 @@ struct EdgeResolver {
       bool ok = true;
       for (int xs = 0; xs < 2; xs++)
          for (int ys = 0; ys < 2; ys++)
-            ok &= line(b, 2, g.nz, [&](int t) { return Cell{b, X[xs], Y[ys], t + 1}; }, fold,
-                       out[xs * 2 + ys]);
+            ok &= line(Cell{b, X[xs], Y[ys], 1}, 2, g.nz, fold, out[xs * 2 + ys]);
       for (int xs = 0; xs < 2; xs++)
          for (int zs = 0; zs < 2; zs++)
-            ok &= line(b, 1, g.ny, [&](int t) { return Cell{b, X[xs], t + 1, Z[zs]}; }, fold,
-                       out[4 + xs * 2 + zs]);
+            ok &= line(Cell{b, X[xs], 1, Z[zs]}, 1, g.ny, fold, out[4 + xs * 2 + zs]);
       for (int ys = 0; ys < 2; ys++)
          for (int zs = 0; zs < 2; zs++)
-            ok &= line(b, 0, g.nx, [&](int t) { return Cell{b, t + 1, Y[ys], Z[zs]}; }, fold,
-                       out[8 + ys * 2 + zs]);
+            ok &= line(Cell{b, 1, Y[ys], Z[zs]}, 0, g.nx, fold, out[8 + ys * 2 + zs]);
       for (int xs = 0; xs < 2; xs++)
          for (int ys = 0; ys < 2; ys++)
             for (int zs = 0; zs < 2; zs++)
-               ok &= line(b, -1, 1, [&](int) { return Cell{b, X[xs], Y[ys], Z[zs]}; }, fold,
-                          out[12 + xs * 4 + ys * 2 + zs]);
+               ok &= line(Cell{b, X[xs], Y[ys], Z[zs]}, -1, 1, fold, out[12 + xs * 4 + ys * 2 + zs]);
       return ok;
    }
 };
@@ -604,6 +618,8 @@ static void face_sources(const amr_dev *d, const int32_t *sorted, int n_active,
       for (size_t i = 0; i < 6 * (size_t) n_active; i++)
          if (P.redir[i] >= 0)
             P.faces[i] = FaceSrc{FS_SAME, {P.redir[i], -1, -1, -1}};
+         else if (P.redir[i] == kRedirBc)
+            P.faces[i].kind = FS_BC;
       return;
    }
    std::vector<int32_t> at(d->c.max_blocks, -1);   // slot -> place in sorted
@@ -643,31 +659,43 @@ static void compute_fused_plan(const amr_dev *d, const int32_t *sorted, int n_ac
                                const amr_face_job *jobs, const int32_t count[3], FusedPlan &P)
 {
    const int M = d->c.max_blocks;
-   std::vector<int32_t> same(6 * (size_t) M, -1);
-   std::vector<uint8_t> bc(M, 0);
+   std::vector<int32_t> kind(6 * (size_t) M, FK_NONE);
+   std::vector<uint8_t> bc(M, 0), quarters(6 * (size_t) M, 0);
    const int nj = count[0] + count[1] + count[2];
+   bool fold = d->g.stencil == 27 && fold_edges_on();
    for (int t = 0; t < nj; t++) {
       const amr_face_job &j = jobs[t];
-      if (j.kind == AMR_FACE_BC)
+      const size_t at = 6 * (size_t) j.dst + j.face;
+      if (j.kind == AMR_FACE_BC) {
          bc[j.dst] = 1;
-      else if (j.kind == AMR_FACE_SAME)
-         same[6 * (size_t) j.dst + j.face] = j.src;
+         kind[at] = FK_BC;
+      } else if (j.kind == AMR_FACE_SAME) {
+         kind[at] = j.src;
+      } else {
+         kind[at] = FK_CF;
+         quarters[at] |= j.kind == AMR_FACE_PROLONG ? 15 : 1 << (j.iq + 2 * j.jq);
+         fold &= !(j.kind & AMR_FACE_GHOSTS);
+      }
    }
-   auto inplace = [&](int slot, int f) { return bc[slot] ? -1 : same[6 * (size_t) slot + f]; };
-   // the in-place faces of each slot (those of boundary blocks are not)
-   std::vector<int32_t> inp(6 * (size_t) M, -1);
-   for (int in = 0; in < n_active; in++)
-      for (int f = 0; f < 6; f++)
-         inp[6 * (size_t) sorted[in] + f] = inplace(sorted[in], f);
+   // folding expects whole coarse/fine planes
+   for (size_t at = 0; at < kind.size() && fold; at++)
+      fold = kind[at] != FK_CF || quarters[at] == 15;
+   // Faces read in place: same-level ones and, when edges are folded, the
+   // boundary's.  Without folding the jobs of a boundary block all run: a
+   // boundary fill with the 27-point extension reads the block's own ghost
+   // planes as they were before the later phases of the stage.
+   auto inplace = [&](int slot, int f) {
+      const int k = kind[6 * (size_t) slot + f];
+      return fold ? (k == FK_CF ? FK_NONE : k) : (bc[slot] || k < 0) ? -1 : k;
+   };
    // edge sources of every active block: folded (27-point stencil) unless a
    // line is not one affine run, in which case the plan keeps the extensions
    std::vector<EdgeSrc> &edges = P.edges;
    edges.assign(kEdgeSrcs * (size_t) M, EdgeSrc{0, 0, 0, ES_ABS});
-   bool fold = d->g.stencil == 27 && fold_edges_on();
    {
       // the blocks are independent: spread them over a few host threads
       // (the resolution takes ~2 ms for 5,500 blocks on one)
-      const EdgeResolver R(d->g, inp, bc);
+      const EdgeResolver R(d->g, kind);
       auto resolve_range = [&](int i0, int i1, bool f) {
          bool ok = true;
          for (int in = i0; in < i1; in++)
@@ -700,7 +728,8 @@ static void compute_fused_plan(const amr_dev *d, const int32_t *sorted, int n_ac
    // cells, which no job writes, and write ghost cells that only later
    // phases' jobs (27-point rings) and the stencil read -- an x job reads
    // ghost cells only in a boundary fill of its own block.  The y and z
-   // launches keep the jobs that read rings.
+   // launches keep the jobs that read rings -- none when edges are folded:
+   // then only coarse/fine jobs are left and one launch holds them all.
    std::vector<FusedJob> ph[3];
    const bool hoist = hoist_on();
    for (int t = 0, dir = 0; dir < 3; dir++)
@@ -710,11 +739,17 @@ static void compute_fused_plan(const amr_dev *d, const int32_t *sorted, int n_ac
          f.jb = j;
          f.mode = FJ_FULL;
          f.alt[0] = f.alt[1] = f.alt[2] = f.alt[3] = -1;
-         f.pad = 0;
+         f.ring = 0;
+         if (fold && (j.kind == AMR_FACE_SAME || j.kind == AMR_FACE_BC))
+            continue;                       // read where it is, edges included
+         if (fold && dir > 0) {
+            // boundary faces of earlier phases beside this coarse/fine plane
+            for (int f2 = 0; f2 < 2 * dir; f2++)
+               f.ring |= (kind[6 * (size_t) j.dst + f2] == FK_BC) << f2;
+         }
          if (j.kind == AMR_FACE_SAME && inplace(j.dst, j.face) >= 0) {
-            if (dir == 0 || d->g.stencil == 7 || fold)
-               continue;                    // nothing outside the face interior, or
-                                            // the extension is read where it is
+            if (dir == 0 || d->g.stencil == 7)
+               continue;                    // nothing outside the face interior
             f.mode = FJ_EXT_ONLY;
          }
          if (d->g.stencil == 27 && dir > 0 &&
@@ -727,14 +762,14 @@ static void compute_fused_plan(const amr_dev *d, const int32_t *sorted, int n_ac
             }
          }
          const bool cf = j.kind == AMR_FACE_PROLONG || j.kind == AMR_FACE_RESTRICT;
-         ph[hoist && dir > 0 && cf && !bc[j.dst] ? 0 : dir].push_back(f);
+         ph[hoist && dir > 0 && cf && (fold || !bc[j.dst]) ? 0 : dir].push_back(f);
       }
    // the jobs that bring stale ghost planes up to date (amr_require_fresh)
    std::vector<amr_face_job> &mj = P.mj;
    int32_t *mc = P.mc;
    for (int t = 0, dir = 0; dir < 3; dir++)
       for (int e = 0; e < count[dir]; e++, t++)
-         if (jobs[t].kind == AMR_FACE_SAME && inplace(jobs[t].dst, jobs[t].face) >= 0) {
+         if (!fold && jobs[t].kind == AMR_FACE_SAME && inplace(jobs[t].dst, jobs[t].face) >= 0) {
             mj.push_back(jobs[t]);
             mc[dir]++;
          }
@@ -747,20 +782,98 @@ static void compute_fused_plan(const amr_dev *d, const int32_t *sorted, int n_ac
    P.redir.assign(6 * (size_t) std::max(n_active, 1), -1);
    for (int in = 0; in < n_active; in++)
       for (int f = 0; f < 6; f++)
-         P.redir[6 * (size_t) in + f] = inplace(sorted[in], f);
+         P.redir[6 * (size_t) in + f] = inplace(sorted[in], f);   // FK_BC: kRedirBc
    face_sources(d, sorted, n_active, jobs, nj, P);
 }
 
 // A fused stage leaves unwritten the ghost cells its stencil reads where
-// they are: the planes of the faces read in place and their 27-point edge
-// extensions, which are exactly what the same-level jobs of blocks without
-// a boundary face write (every other job runs in the fused stage).  The
-// interiors those jobs read in the plain stage are the ones the fused stage
-// read, which the record still holds in its other interior copy until the
-// next stage writes it; a job's reads of other ghost cells find them as the
-// plain stage's earlier phases left them (written by the fused stage, or by
-// this rerun's earlier directions).  So rerunning those jobs, in direction
-// order, on the other copy gives every ghost cell the plain stage's value.
+// they are.  The interiors it read them from are still in the record's other
+// copy, until the next stage writes it.
+//   Edges folded: every such cell is in the tables -- the planes of the faces
+// read in place (redir) and the edge entries -- and their sources are
+// interior cells, coarse/fine ghost cells and stale edge cells, none of which
+// is filled here, so one launch copies them all (k_fill_in_place).
+//   Otherwise they are what the same-level jobs of blocks without a boundary
+// face write (7-point stages that read every face in place: all jobs).  A
+// job's reads of other ghost cells find them as the plain stage's earlier
+// phases left them, so rerunning those jobs, in direction order, on the other
+// copy gives every ghost cell the plain stage's value.
+template <typename T>
+static __global__ __launch_bounds__(256) void k_fill_in_place(
+   T *__restrict__ pool, const int32_t *__restrict__ sorted, const int32_t *__restrict__ redir,
+   const EdgeSrc *__restrict__ edges, Lay L, int var0)
+{
+   const int slot = sorted[blockIdx.x];
+   T *const var = pool + (int64_t) (var0 + blockIdx.y) * L.var_stride;
+   T *const rec = var + (int64_t) slot * L.rec;
+   auto fill = [&](int i, int j, int k, T v) {
+      rec[home(L, i, j, k)] = v;
+      if (k == 1 || k == L.nz)
+         rec[zcopy(L, i, j, k)] = v;
+   };
+   for (int f = 0; f < 6; f++) {
+      const int from = redir[6 * (int64_t) blockIdx.x + f];
+      if (from == -1)
+         continue;
+      const int dir = f >> 1, hi = f & 1, n = dir == 0 ? L.nx : dir == 1 ? L.ny : L.nz;
+      const int na = dir == 0 ? L.ny : L.nx, nb = dir == 2 ? L.ny : L.nz;
+      const bool own = from == kRedirBc;   // the block's own plane next to the face
+      const T *const src = own ? rec : var + (int64_t) from * L.rec;
+      const int ghost = hi ? n + 1 : 0, plane = own == (hi != 0) ? n : 1;
+      for (int t = threadIdx.x; t < na * nb; t += blockDim.x) {
+         const int a = 1 + t / nb, b = 1 + t % nb;
+         const int i = dir == 0 ? ghost : a, j = dir == 0 ? a : dir == 1 ? ghost : b,
+                   k = dir == 2 ? ghost : b;
+         const int si = dir == 0 ? plane : i, sj = dir == 1 ? plane : j, sk = dir == 2 ? plane : k;
+         fill(i, j, k, src[dir == 2 ? zcopy(L, si, sj, sk) : home(L, si, sj, sk)]);
+      }
+   }
+   const EdgeSrc *const es = edges + (int64_t) kEdgeSrcs * slot;
+   const int nz4 = 4 * L.nz, ny4 = 4 * L.ny, nx4 = 4 * L.nx;
+   for (int e = threadIdx.x; e < nz4 + ny4 + nx4 + 8; e += blockDim.x) {
+      int i, j, k, line, t;
+      if (e < nz4) {
+         line = e / L.nz; t = e - line * L.nz;
+         i = (line & 2) ? L.nx + 1 : 0; j = (line & 1) ? L.ny + 1 : 0; k = t + 1;
+      } else if (e < nz4 + ny4) {
+         const int h = e - nz4;
+         line = h / L.ny; t = h - line * L.ny;
+         i = (line & 2) ? L.nx + 1 : 0; k = (line & 1) ? L.nz + 1 : 0; j = t + 1;
+         line += 4;
+      } else if (e < nz4 + ny4 + nx4) {
+         const int h = e - nz4 - ny4;
+         line = h / L.nx; t = h - line * L.nx;
+         j = (line & 2) ? L.ny + 1 : 0; k = (line & 1) ? L.nz + 1 : 0; i = t + 1;
+         line += 8;
+      } else {
+         const int h = e - nz4 - ny4 - nx4;
+         line = 12 + h; t = 0;
+         i = (h & 4) ? L.nx + 1 : 0; j = (h & 2) ? L.ny + 1 : 0; k = (h & 1) ? L.nz + 1 : 0;
+      }
+      const int64_t from = edge_at(es[line], L, t);
+      if (from != (int64_t) slot * L.rec + home(L, i, j, k))
+         fill(i, j, k, var[from]);
+   }
+}
+
+static int launch_fill_in_place(amr_dev *d, const Lay &L, int start, int num)
+{
+   if (!d->n_active)
+      return AMR_OK;
+   const dim3 grid(d->n_active, num);
+   if (d->elem_bytes == 8)
+      hipLaunchKernelGGL(k_fill_in_place<uint64_t>, grid, dim3(256), 0, d->stream,
+                         (uint64_t *) d->pool, d->d_sorted, d->d_redir, d->d_edges, L, start);
+   else if (d->elem_bytes == 4)
+      hipLaunchKernelGGL(k_fill_in_place<uint32_t>, grid, dim3(256), 0, d->stream,
+                         (uint32_t *) d->pool, d->d_sorted, d->d_redir, d->d_edges, L, start);
+   else
+      hipLaunchKernelGGL(k_fill_in_place<uint16_t>, grid, dim3(256), 0, d->stream,
+                         (uint16_t *) d->pool, d->d_sorted, d->d_redir, d->d_edges, L, start);
+   HIP_TRY(d, hipGetLastError());
+   return AMR_OK;
+}
+
 int amr_require_fresh(amr_dev *d, int start, int num, const char *what)
 {
    const int end = std::min(start + num, (int) d->stale.size());
@@ -776,7 +889,14 @@ int amr_require_fresh(amr_dev *d, int start, int num, const char *what)
       if (int rc = amr_lay(d, a, b - a, &L))
          return rc;
       const Lay Lr = amr_lay_other(d, L);
-      // a stage that read every face in place left every ghost plane
+      if (d->fold_edges) {
+         if (int rc = launch_fill_in_place(d, Lr, a, b - a))
+            return rc;
+         for (int v = a; v < b; v++)
+            d->stale[v] = 0;
+         a = b;
+         continue;
+      }
       const amr_face_job *jobs = d->all_faces ? d->d_jobs : d->d_mjobs;
       const int32_t *cnt = d->all_faces ? d->count : d->mcount;
       for (int dir = 0, off = 0; dir < 3; off += cnt[dir], dir++)
@@ -868,7 +988,7 @@ int amr_set_mesh_impl(amr_dev *d, const int32_t *sorted, int n_active,
          HIP_TRY(d, hipMalloc(&d->d_edges, sizeof(EdgeSrc) * fp.edges.size()));
       if (!d->d_redir)
          HIP_TRY(d, hipMalloc(&d->d_redir, sizeof(int32_t) * 6 * (size_t) d->c.max_blocks));
-      if (!d->d_faces)
+      if (!d->d_faces && !fp.faces.empty())
          HIP_TRY(d, hipMalloc(&d->d_faces, sizeof(FaceSrc) * 6 * (size_t) d->c.max_blocks));
    }
    // One pinned staging buffer, then copies ordered on the stream before
@@ -1324,19 +1444,21 @@ int amr_dev_stage_fused(amr_dev *d, int start, int num, int stage, int permute, 
 {
    if (!d)
       return AMR_ERR_ARG;
-   // the plain stage where in-place reads cannot stand in for it (permuted
-   // phases, --code 1/2 planes, taping and replay), and for
-   // stages below ~1e8 cell updates: those are bound by launch latency,
-   // where the fused kernels' longer set-up costs more than the ghost planes
-   // they save (FP32 runs of 8^3-16^3 blocks with 8-40 variables measured
-   // 1-7% slower fused; the 16^3, 40-variable bandwidth-scale run 15-18%
-   // faster)
+   // The plain stage where in-place reads cannot stand in for it (permuted
+   // phases, --code 1/2 planes, taping and replay, jobs on inactive blocks),
+   // and below ~1e8 cell updates where the fused stage still needs the three
+   // ordered exchange launches (edges not folded): such stages are bound by
+   // launch latency, where the fused kernels' longer set-up costs more than
+   // the ghost planes they save (1-7% slower).  With folded edges a stage is
+   // one coarse/fine launch and the stencil at most: 60 blocks of 6x10x14 in
+   // FP32 take 2.6 ms for 200 stages against 5.6 ms plain, the moving-object
+   // run (16^3, 12 variables) 32.5 ms against 35.4.
    const double cells = (double) d->n_active * num * d->g.nx * d->g.ny * d->g.nz;
    // a 7-point stage that reads every face in place is one launch at any size,
    // and the order of the phases does not matter to it
    if (!d->two_interiors || !d->closed || (permute && !d->all_faces) || d->whole_ghosts ||
        (d->tape && d->tape->on) || d->replaying ||
-       (d->fused_mode == 1 && cells < 1.0e8 && !d->all_faces))
+       (d->fused_mode == 1 && cells < 1.0e8 && !d->all_faces && !d->fold_edges))
       return amr_dev_stage(d, start, num, stage, permute, sum_row);
    if (start < 0 || num < 0 || start + num > d->c.num_vars)
       return amr_set_error(d, AMR_ERR_ARG, "stage: variables out of range");

@@ -278,6 +278,46 @@ __device__ __forceinline__ void exchange_job(T *__restrict__ pool, const amr_fac
    }
 }
 
+// The ring cells beside a coarse/fine ghost plane that a boundary fill of an
+// earlier direction copied from it (FusedJob::ring): they take the plane's
+// present cells, before the job writes the new ones -- every thread of the
+// item has read its cells when the function returns.
+template <typename T>
+__device__ __forceinline__ void keep_ring(T *__restrict__ pool, const FusedJob &fj, const Lay &L,
+                                          int v0, int nv, int tid, int nthr)
+{
+   const amr_face_job &jb = fj.jb;
+   const int dir = jb.face >> 1, n = dir == 1 ? L.ny : L.nz, ghost = (jb.face & 1) ? n + 1 : 0;
+   const int na = L.nx, nb = dir == 2 ? L.ny : L.nz;   // dir 1: (x, z), dir 2: (x, y)
+   const bool quarter = jb.kind == AMR_FACE_RESTRICT;
+   T *const rec = pool + (int64_t) v0 * L.var_stride + (int64_t) jb.dst * L.rec;
+   for (int t = tid; t < 2 * (na + nb); t += nthr) {
+      // faces W, E (the rows a = 1, na) and, for a z plane, S, N (b = 1, nb)
+      const int f = t < nb ? 0 : t < 2 * nb ? 1 : t < 2 * nb + na ? 2 : 3;
+      if (!(fj.ring >> f & 1))
+         continue;
+      const int a = f == 0 ? 1 : f == 1 ? na : t - 2 * nb - (f - 2) * na + 1;
+      const int b = f < 2 ? t - f * nb + 1 : f == 2 ? 1 : nb;
+      if (quarter && ((a > na / 2) != (jb.jq != 0) || (b > nb / 2) != (jb.iq != 0)))
+         continue;
+      int i, j, k, ri, rj, rk;
+      canon(dir, ghost, a, b, i, j, k);
+      canon(dir, ghost, f == 0 ? 0 : f == 1 ? na + 1 : a, f == 2 ? 0 : f == 3 ? nb + 1 : b, ri, rj,
+            rk);
+      const int so = home(L, i, j, k), dh = home(L, ri, rj, rk);
+      const int dc = rk == 1 || rk == L.nz ? zcopy(L, ri, rj, rk) : -1;
+      for (int q = 0; q < nv; q++) {
+         T *const r = rec + q * L.var_stride;
+         const T v = r[so];
+         r[dh] = v;
+         if (dc >= 0)
+            r[dc] = v;
+      }
+   }
+   if (nthr > 64)
+      __syncthreads();
+}
+
 // One face job of a fused stage (FusedJob).  Prolongation and restriction
 // are the plain fill.  Same-level and boundary jobs fill their cells as the
 // plain fill does, except that an FJ_EXT_ONLY job fills only the cells
@@ -298,6 +338,8 @@ __device__ __forceinline__ void exchange_job_fused(T *__restrict__ pool, const F
    const amr_face_job &jb = fj.jb;
    if (jb.kind == AMR_FACE_PROLONG || jb.kind == AMR_FACE_RESTRICT ||
        (jb.kind & AMR_FACE_GHOSTS)) {
+      if (fj.ring)
+         keep_ring<T>(pool, fj, L, v0, nv, tid, nthr);
       exchange_job<T, KV>(pool, jb, L, v0, nv, tid, nthr);
       return;
    }

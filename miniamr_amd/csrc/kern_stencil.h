@@ -120,9 +120,9 @@ template <typename T> __device__ __forceinline__ T load_at(gptr<T> b, int64_t o)
 // then become constants); 0 reads it from L.  D planes of loads are kept
 // in flight (small blocks can afford all of theirs).
 //
-// FUSED (a stage that reads same-level faces in place): the block's slot
-// bslot, redir[6], the slots its six faces are read from (-1: its own ghost
-// plane), and es[kEdgeSrcs], where its ghost edge lines and corners are
+// FUSED (a stage that reads same-level and boundary faces in place): the
+// block's slot bslot, redir[6], the slots its six faces are read from (-1: its
+// own ghost plane; kRedirBc: its own plane next to the face), and es[kEdgeSrcs], where its ghost edge lines and corners are
 // read (EdgeSrc).  The face interior of a redirected face is read from the
 // neighbour's interior (its z-plane copy for z faces) in the copy L
 // describes, and the outputs go to the copy Lout describes, so no
@@ -197,10 +197,12 @@ __device__ __forceinline__ void stencil_block(T *__restrict__ rec, const Lay &L,
          const int64_t own = (int64_t) bslot * L.rec;
          const bool jin = jj >= 1 && jj <= L.ny, kin = kk >= 1 && kk <= nz;
          if (jin && kin) {
-            off0[q] = rdr[0] >= 0 ? (int64_t) rdr[0] * L.rec + home(L, L.nx, jj, kk)
-                                  : own + home(L, 0, jj, kk);
-            offN[q] = rdr[1] >= 0 ? (int64_t) rdr[1] * L.rec + home(L, 1, jj, kk)
-                                  : own + home(L, L.nx + 1, jj, kk);
+            off0[q] = rdr[0] >= 0          ? (int64_t) rdr[0] * L.rec + home(L, L.nx, jj, kk)
+                      : rdr[0] == kRedirBc ? own + home(L, 1, jj, kk)
+                                           : own + home(L, 0, jj, kk);
+            offN[q] = rdr[1] >= 0          ? (int64_t) rdr[1] * L.rec + home(L, 1, jj, kk)
+                      : rdr[1] == kRedirBc ? own + home(L, L.nx, jj, kk)
+                                           : own + home(L, L.nx + 1, jj, kk);
          } else {
             // an edge line or corner of the x = 0 / x = nx+1 planes (the
             // x = nx+1 entry follows the x = 0 one at +2, corners at +4)
@@ -221,22 +223,18 @@ __device__ __forceinline__ void stencil_block(T *__restrict__ rec, const Lay &L,
             b = edge_at(x, L, 0);
             o1 = 0;
             o2 = x.stride;
-         } else if (kin && jj == 0 && rdr[2] >= 0) {
-            b = (int64_t) rdr[2] * L.rec;
-            o1 = home(L, 1, L.ny, kk);
-            o2 = L.nx > 1 ? home(L, 2, L.ny, kk) : o1;
-         } else if (kin && jj == L.ny + 1 && rdr[3] >= 0) {
-            b = (int64_t) rdr[3] * L.rec;
-            o1 = home(L, 1, 1, kk);
-            o2 = L.nx > 1 ? home(L, 2, 1, kk) : o1;
-         } else if (jin && kk == 0 && rdr[4] >= 0) {
-            b = (int64_t) rdr[4] * L.rec;
-            o1 = zcopy(L, 1, jj, nz);
-            o2 = L.nx > 1 ? zcopy(L, 2, jj, nz) : o1;
-         } else if (jin && kk == nz + 1 && rdr[5] >= 0) {
-            b = (int64_t) rdr[5] * L.rec;
-            o1 = zcopy(L, 1, jj, 1);
-            o2 = L.nx > 1 ? zcopy(L, 2, jj, 1) : o1;
+         } else if (jin != kin) {
+            // the face this row belongs to, the slot it is read from (a
+            // boundary face: the block's own) and that block's row
+            const int f = kin ? (jj == 0 ? 2 : 3) : kk == 0 ? 4 : 5;
+            const int from = f == 2 ? rdr[2] : f == 3 ? rdr[3] : f == 4 ? rdr[4] : rdr[5];
+            if (from != -1) {
+               const bool bnd = from == kRedirBc;
+               const int n = f < 4 ? L.ny : nz, row = (f & 1) != (int) bnd ? 1 : n;
+               b = bnd ? own : (int64_t) from * L.rec;
+               o1 = f < 4 ? home(L, 1, row, kk) : zcopy(L, 1, jj, row);
+               o2 = L.nx > 1 ? (f < 4 ? home(L, 2, row, kk) : zcopy(L, 2, jj, row)) : o1;
+            }
          }
          off1[q] = b + o1;
          stp[q] = o2 - o1;

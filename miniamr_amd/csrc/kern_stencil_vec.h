@@ -109,9 +109,12 @@ __device__ __forceinline__ void stencil27_v16(T *__restrict__ rec, const Lay &L,
    // the thread's interior vector: plane 0, plane nx+1, plane 1 (then +NCOL)
    Off iv0, ivN, iv1;
    if constexpr (FUSED) {
-      iv0 = rdr[0] >= 0 ? (int64_t) rdr[0] * L.rec + home(L, L.nx, j, k0) : own + home(L, 0, j, k0);
-      ivN = rdr[1] >= 0 ? (int64_t) rdr[1] * L.rec + home(L, 1, j, k0)
-                        : own + home(L, L.nx + 1, j, k0);
+      iv0 = rdr[0] >= 0          ? (int64_t) rdr[0] * L.rec + home(L, L.nx, j, k0)
+            : rdr[0] == kRedirBc ? own + home(L, 1, j, k0)
+                                 : own + home(L, 0, j, k0);
+      ivN = rdr[1] >= 0          ? (int64_t) rdr[1] * L.rec + home(L, 1, j, k0)
+            : rdr[1] == kRedirBc ? own + home(L, L.nx, j, k0)
+                                 : own + home(L, L.nx + 1, j, k0);
    } else {
       iv0 = home(L, 0, j, k0);
       ivN = home(L, L.nx + 1, j, k0);
@@ -163,22 +166,18 @@ __device__ __forceinline__ void stencil27_v16(T *__restrict__ rec, const Lay &L,
             b = edge_at(x, L, 0);
             o1 = 0;
             o2 = x.stride;
-         } else if (jj == 0 && rdr[2] >= 0) {
-            b = (int64_t) rdr[2] * L.rec;
-            o1 = home(L, 1, N, kk);
-            o2 = L.nx > 1 ? home(L, 2, N, kk) : o1;
-         } else if (jj == G - 1 && rdr[3] >= 0) {
-            b = (int64_t) rdr[3] * L.rec;
-            o1 = home(L, 1, 1, kk);
-            o2 = L.nx > 1 ? home(L, 2, 1, kk) : o1;
-         } else if (kk == 0 && rdr[4] >= 0) {
-            b = (int64_t) rdr[4] * L.rec;
-            o1 = zcopy(L, 1, jj, N);
-            o2 = L.nx > 1 ? zcopy(L, 2, jj, N) : o1;
-         } else if (kk == G - 1 && rdr[5] >= 0) {
-            b = (int64_t) rdr[5] * L.rec;
-            o1 = zcopy(L, 1, jj, 1);
-            o2 = L.nx > 1 ? zcopy(L, 2, jj, 1) : o1;
+         } else {
+            // the face this row belongs to, the slot it is read from (a
+            // boundary face: the block's own) and that block's row
+            const int f = jj == 0 ? 2 : jj == G - 1 ? 3 : kk == 0 ? 4 : 5;
+            const int from = f == 2 ? rdr[2] : f == 3 ? rdr[3] : f == 4 ? rdr[4] : rdr[5];
+            if (from != -1) {
+               const bool bnd = from == kRedirBc;
+               const int row = (f & 1) != (int) bnd ? 1 : N;
+               b = bnd ? own : (int64_t) from * L.rec;
+               o1 = f < 4 ? home(L, 1, row, kk) : zcopy(L, 1, jj, row);
+               o2 = L.nx > 1 ? (f < 4 ? home(L, 2, row, kk) : zcopy(L, 2, jj, row)) : o1;
+            }
          }
          r1[q] = vo + b + o1;
          rstp[q] = o2 - o1;

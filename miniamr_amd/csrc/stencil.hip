@@ -59,8 +59,9 @@ __global__ __launch_bounds__(kThreads) void k_stencil(T *__restrict__ pool,
 }
 
 // The stencil of a fused stage: interiors read from the copy L describes,
-// written to the copy Lo describes, same-level faces read in place through
-// redir (six slots per active block, sorted order), ghost edge lines and
+// written to the copy Lo describes, same-level and boundary faces read in place
+// through redir (six entries per active block, sorted order: the slot,
+// kRedirBc or -1), ghost edge lines and
 // corners where edges (kEdgeSrcs entries per slot) says.
 template <typename T, int ST, int NC, int NP, int V, int NZ>
 __global__ __launch_bounds__(kThreads) void k_stencil_fused(T *__restrict__ pool,
