@@ -579,13 +579,14 @@ struct EdgeResolver {
 
 }  // namespace
 
-// The plan of amr_dev_stage_fused.  A block's face is read in place when
-// its job is a same-level copy and the block has no boundary face (a
-// boundary fill with the 27-point extension reads the block's own ghost
-// planes as they were before the later phases of the stage, which an
-// in-place read cannot reproduce).  Such a face's job is dropped (x, and
-// y/z for the 7-point stencil) or reduced to its edge extension (y/z for
-// the 27-point stencil); every job that reads a source's ghost row that is
+// The plan of amr_dev_stage_fused.  Edges folded (27-point): same-level and
+// boundary faces are read in place, edges through the entries above, and only
+// coarse/fine jobs remain.  Otherwise a face is read in place when its job is
+// a same-level copy and the block has no boundary face (a boundary fill with
+// the 27-point extension reads the block's own ghost planes as they were
+// before the later phases of the stage); such a face's job is dropped (x, and
+// y/z for the 7-point stencil) or reduced to its edge extension (y/z for the
+// 27-point stencil), and every job that reads a source's ghost row that is
 // read in place is redirected to the block that row would be copied from.
 // It is computed on the host only; set_mesh uploads it.
 struct FusedPlan {

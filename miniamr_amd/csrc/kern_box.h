@@ -12,6 +12,12 @@
 // block: a variable costs a thread its loads (one scalar base per variable and
 // 32-bit offsets that do not change), the LDS traffic and the sums.
 //
+// Measured: 890 blocks of 10^3 x 40 variables, FP64, a 7-point stage 365 us
+// (three exchange launches and the stencil) -> 150 us, bound by its traffic
+// (28.7 KB per block-variable of 16 KB algorithmic: ghost planes, z-plane
+// copies, 80-byte rows in 128-byte lines) and the workgroups in flight; 64
+// blocks of 8^3 x 4 variables 23 -> 5 us, bound by the launch.
+//
 // Faces.  A ghost plane is read from where its values come from (FaceSrc): the
 // block's own plane, a same-level neighbour's interior, the block's own
 // boundary plane, a coarse neighbour's cells / 4 or sums of four fine cells,
