@@ -467,7 +467,7 @@ void amr_tape_record(amr_dev *d, int kind, int a1 = 0, int a2 = 0, int a3 = 0, i
 void amr_tape_free(amr_dev *d);
 
 // The layout of variables [start, start+num) with their current interior
-// copy (AMR_ERR_STATE, via amr_set_error, if the range mixes copies).
+// copy (brought to one copy first if fused stages left them in two).
 int amr_lay(amr_dev *d, int start, int num, Lay *out);
 // The same layout with the other interior copy (where a stage writes).
 Lay amr_lay_other(const amr_dev *d, const Lay &L);

@@ -272,17 +272,16 @@ int amr_dev_download_block(amr_dev *d, int slot, double *cells)
 
 }  // extern "C"
 
+static int unify_copies(amr_dev *d, int start, int num);
+
 int amr_lay(amr_dev *d, int start, int num, Lay *out)
 {
    *out = d->g;
    if (num <= 0)
       return AMR_OK;
+   if (int rc = unify_copies(d, start, num))
+      return rc;
    const int p = d->par[start];
-   for (int v = start + 1; v < start + num; v++)
-      if (d->par[v] != p)
-         return amr_set_error(d, AMR_ERR_STATE,
-                              "variables %d and %d hold their cells in different copies",
-                              start, v);
    out->oI = d->oI_par[p];
    out->oZI = d->oZI_par[p];
    return AMR_OK;
@@ -364,6 +363,25 @@ static void add_moves(std::vector<CopyMove> &mv, int slot, const uint8_t *is, co
          mv.push_back({slot, v, e - v, is[v]});
       v = e;
    }
+}
+
+// Bring the cells of variables [start, start+num) to one interior copy, the
+// first variable's: fused stages of single variables leave them in different
+// ones, and a launch works on one.  A variable's stale ghost planes are filled
+// first, from the copy that the move then overwrites.
+static int unify_copies(amr_dev *d, int start, int num)
+{
+   std::vector<CopyMove> mv;
+   for (int v = start + 1; v < start + num; v++) {
+      if (d->par[v] == d->par[start])
+         continue;
+      if (int rc = amr_require_fresh(d, v, 1, "variables in different copies"))
+         return rc;
+      for (int s : d->h_sorted)
+         mv.push_back({s, v, 1, d->par[v]});
+      d->par[v] = d->par[start];
+   }
+   return move_copies(d, mv);
 }
 
 void amr_slot_written(amr_dev *d, int slot)

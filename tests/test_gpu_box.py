@@ -64,6 +64,14 @@ def test_stages_match(n, st, prec, monkeypatch):
     np.testing.assert_allclose(g.read_sums(0, 3), c.read_sums(0, 3), rtol=1e-13)
     for s in range(11):
         assert np.array_equal(g.download(s), c.download(s)), s
+    # some variables one stage ahead: read them, then go on with all of them
+    for k, (start, num) in enumerate([(0, 1), (0, nv), (1, 2), (0, nv)]):
+        g.stage_fused(start, num, stage=k)
+        c.stage(start, num, stage=k)
+        if k < 3:
+            assert np.array_equal(g.download(order[k]), c.download(order[k])), k
+    for s in range(11):
+        assert np.array_equal(g.download(s), c.download(s)), s
 
 
 def test_inactive_slots_and_saved_states():
