@@ -281,7 +281,10 @@ __device__ __forceinline__ void exchange_job(T *__restrict__ pool, const amr_fac
 // The ring cells beside a coarse/fine ghost plane that a boundary fill of an
 // earlier direction copied from it (FusedJob::ring): they take the plane's
 // present cells, before the job writes the new ones -- every thread of the
-// item has read its cells when the function returns.
+// item has read its cells when the function returns.  An item of one
+// wavefront has no barrier: the fences keep the compiler from moving one
+// lane's loads past the stores that other lanes make to the same cells
+// afterwards (a wavefront's accesses to one address stay in program order).
 template <typename T>
 __device__ __forceinline__ void keep_ring(T *__restrict__ pool, const FusedJob &fj, const Lay &L,
                                           int v0, int nv, int tid, int nthr)
@@ -314,8 +317,13 @@ __device__ __forceinline__ void keep_ring(T *__restrict__ pool, const FusedJob &
             r[dc] = v;
       }
    }
-   if (nthr > 64)
+   if (nthr > 64) {
       __syncthreads();
+   } else {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+   }
 }
 
 // One face job of a fused stage (FusedJob).  Prolongation and restriction
