@@ -244,6 +244,7 @@ struct amr_dev {
    // slot was last written or active ([slot][variable]; two interiors only).
    std::vector<uint8_t> slot_par;
    std::vector<uint8_t> active;     // per slot: in the active list (two interiors only)
+   std::vector<int32_t> inactive_src;   // slots outside it that the plan's jobs read
    bool group_lds_set = false;      // k_mat_group's LDS limit raised
 };
 
@@ -467,8 +468,13 @@ void amr_tape_record(amr_dev *d, int kind, int a1 = 0, int a2 = 0, int a3 = 0, i
 void amr_tape_free(amr_dev *d);
 
 // The layout of variables [start, start+num) with their current interior
-// copy (brought to one copy first if fused stages left them in two).
+// copy (AMR_ERR_STATE, via amr_set_error, if the range mixes copies: entry
+// points bring it to one with amr_unify before they look at slots).
 int amr_lay(amr_dev *d, int start, int num, Lay *out);
+// Bring the cells of variables [start, start+num) to one interior copy if
+// fused stages of some of them left them in two.  It changes par, so it comes
+// before any comparison or record of a slot's copies.
+int amr_unify(amr_dev *d, int start, int num);
 // The same layout with the other interior copy (where a stage writes).
 Lay amr_lay_other(const amr_dev *d, const Lay &L);
 

@@ -440,6 +440,8 @@ int ensure_table(amr_batch *b)
       m.sorted = d->d_sorted;
       m.partials = d->d_partials;
       m.sums = d->d_sums;
+      if (int rc = amr_unify(d, 0, d->c.num_vars))
+         return berr(b, rc, "member %d: %s", q, d->err);
       if (int rc = amr_lay(d, 0, d->c.num_vars, &m.L))
          return berr(b, rc, "member %d: %s", q, d->err);
       m.Lo = amr_lay_other(d, m.L);

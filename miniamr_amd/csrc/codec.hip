@@ -302,6 +302,8 @@ int codec(amr_dev *d, bool pack, int code, int dir, int start, int num,
          return amr_set_error(d, AMR_ERR_ARG, "%s: message %d ends past the buffer (%zu values)",
                               what, t, buf_elems);
    }
+   if (int rc = amr_unify(d, start, num))
+      return rc;
    for (int t = 0; t < n; t++)
       if (int rc = amr_slots_current(d, &msgs[t].slot, 1))
          return rc;

@@ -86,6 +86,10 @@ extern "C" int amr_dev_compare_cells(amr_dev *a, amr_dev *b, int start, int num,
       return amr_set_error(a, AMR_ERR_STATE, "compare_cells: the contexts hold different "
                            "meshes");
    Lay La, Lb;
+   if (int rc = amr_unify(a, start, num))
+      return rc;
+   if (int rc = amr_unify(b, start, num))
+      return amr_set_error(a, rc, "compare_cells: %s", amr_dev_last_error(b));
    if (int rc = amr_lay(a, start, num, &La))
       return rc;
    if (int rc = amr_lay(b, start, num, &Lb))

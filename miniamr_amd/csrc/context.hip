@@ -235,6 +235,8 @@ int amr_dev_upload_block(amr_dev *d, int slot, const double *cells)
 {
    if (!d || !cells || slot < 0 || slot >= d->c.max_blocks)
       return amr_set_error(d, AMR_ERR_ARG, "upload: slot %d out of range", slot);
+   if (int rc = amr_unify(d, 0, d->c.num_vars))
+      return rc;
    size_t bytes = sizeof(double) * (size_t) d->g.gx * d->g.gy * d->g.gz * d->c.num_vars;
    HIP_TRY(d, hipMemcpyAsync(d->d_stage, cells, bytes, hipMemcpyHostToDevice, d->stream));
    int rc = amr_launch_convert_in(d, slot);
@@ -252,6 +254,8 @@ int amr_dev_download_block(amr_dev *d, int slot, double *cells)
       return AMR_ERR_STATE;
    if (!d || !cells || slot < 0 || slot >= d->c.max_blocks)
       return amr_set_error(d, AMR_ERR_ARG, "download: slot %d out of range", slot);
+   if (int rc = amr_unify(d, 0, d->c.num_vars))
+      return rc;
    if (int rc = amr_slots_current(d, &slot, 1))
       return rc;
    size_t bytes = sizeof(double) * (size_t) d->g.gx * d->g.gy * d->g.gz * d->c.num_vars;
@@ -272,16 +276,17 @@ int amr_dev_download_block(amr_dev *d, int slot, double *cells)
 
 }  // extern "C"
 
-static int unify_copies(amr_dev *d, int start, int num);
-
 int amr_lay(amr_dev *d, int start, int num, Lay *out)
 {
    *out = d->g;
    if (num <= 0)
       return AMR_OK;
-   if (int rc = unify_copies(d, start, num))
-      return rc;
    const int p = d->par[start];
+   for (int v = start + 1; v < start + num; v++)
+      if (d->par[v] != p)
+         return amr_set_error(d, AMR_ERR_STATE,
+                              "variables %d and %d hold their cells in different copies",
+                              start, v);
    out->oI = d->oI_par[p];
    out->oZI = d->oZI_par[p];
    return AMR_OK;
@@ -365,11 +370,12 @@ static void add_moves(std::vector<CopyMove> &mv, int slot, const uint8_t *is, co
    }
 }
 
-// Bring the cells of variables [start, start+num) to one interior copy, the
-// first variable's: fused stages of single variables leave them in different
-// ones, and a launch works on one.  A variable's stale ghost planes are filled
-// first, from the copy that the move then overwrites.
-static int unify_copies(amr_dev *d, int start, int num)
+// The cells of variables [start, start+num) go to the first variable's copy:
+// fused stages of single variables leave them in different ones, and a launch
+// works on one.  A variable's stale ghost planes are filled first, from the
+// copy that the move then overwrites.  The inactive slots that the plan's jobs
+// read were brought to the copies par named when the plan came, and move along.
+int amr_unify(amr_dev *d, int start, int num)
 {
    std::vector<CopyMove> mv;
    for (int v = start + 1; v < start + num; v++) {
@@ -379,6 +385,12 @@ static int unify_copies(amr_dev *d, int start, int num)
          return rc;
       for (int s : d->h_sorted)
          mv.push_back({s, v, 1, d->par[v]});
+      for (int s : d->inactive_src) {
+         uint8_t &is = d->slot_par[(size_t) s * d->c.num_vars + v];
+         if (is == d->par[v])
+            mv.push_back({s, v, 1, d->par[v]});
+         is = d->par[start];
+      }
       d->par[v] = d->par[start];
    }
    return move_copies(d, mv);
@@ -967,14 +979,20 @@ int amr_set_mesh_impl(amr_dev *d, const int32_t *sorted, int n_active,
       for (int i = 0; i < n_active; i++)
          act[sorted[i]] = 1;
       d->closed = true;
+      std::vector<int32_t> outside;   // inactive slots the jobs read, each once
+      std::vector<uint8_t> seen(d->c.max_blocks, 0);
       for (int t = 0; t < nj; t++) {
-         if (!act[jobs[t].src])
-            used.push_back(jobs[t].src);
-         d->closed &= act[jobs[t].src] && act[jobs[t].dst];
+         const int s = jobs[t].src;
+         if (!act[s] && !seen[s])
+            outside.push_back(s);
+         seen[s] = 1;
+         d->closed &= act[s] && act[jobs[t].dst];
       }
+      used.insert(used.end(), outside.begin(), outside.end());
       if (int rc = amr_slots_current(d, used.data(), (int) used.size()))
          return rc;
       d->active.swap(act);
+      d->inactive_src.swap(outside);
    }
    // The fused plan is host work; it runs before the wait below, so it
    // overlaps the device work still queued (split and consolidate data).
@@ -1075,6 +1093,8 @@ int amr_comm_impl(amr_dev *d, int start, int num, int stage, int permute)
                            start + num);
    if (!num)
       return AMR_OK;
+   if (int rc = amr_unify(d, start, num))
+      return rc;
    // one span per direction when timing per direction, else one in all
    if (!d->timing_dirs)
       amr_span_begin(d, 0);
@@ -1243,6 +1263,8 @@ static int refine_slots_current(amr_dev *d, const J *jobs, int n)
 {
    if (!d->two_interiors)
       return AMR_OK;
+   if (int rc = amr_unify(d, 0, d->c.num_vars))
+      return rc;
    std::vector<uint8_t> octants;   // of each merged block, when first needed
    for (int t = 0; t < n; t++) {
       int32_t rd, wr;
@@ -1485,6 +1507,8 @@ int amr_dev_stage_fused(amr_dev *d, int start, int num, int stage, int permute, 
       return amr_set_error(d, AMR_ERR_ARG, "stage: checksum row %d not reserved", sum_row);
    if (!num)
       return AMR_OK;
+   if (int rc = amr_unify(d, start, num))
+      return rc;
    if (!d->timing_dirs && !d->all_faces)
       amr_span_begin(d, 0);
    for (int dir = 0; dir < 3 && !d->all_faces; dir++) {
