@@ -302,6 +302,7 @@ struct amr_batch {
    std::vector<amr_dev *> members;
    std::vector<char> active;
    std::vector<int> seen;            // plan_version of each member at the last build
+   std::vector<int> par;             // the interior copy its cells were in then
 
    // work lists
    BMember *d_mem = nullptr;
@@ -398,14 +399,26 @@ void span_end(amr_batch *b)
 
 int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
-// Rebuild the member table and prefix lists when a member's plan changed,
-// a member joined or left, or the stencil's variables per item changed.
+// A member's cells are still in the interior copy that the table names: its
+// own fused stages and saved or loaded states move them, without a new plan.
+bool cells_in(const amr_dev *d, int copy)
+{
+   for (uint8_t p : d->par)
+      if (p != copy)
+         return false;
+   return true;
+}
+
+// Rebuild the member table and prefix lists when a member's plan changed, its
+// cells moved to the other interior copy, a member joined or left, or the
+// stencil's variables per item changed.
 int ensure_table(amr_batch *b)
 {
    bool need = !b->table_ok || b->table_vpw != b->vpw || b->table_wg != b->wg_mask ||
                b->table_exv != b->ex_vars;
    for (size_t i = 0; i < b->members.size() && !need; i++)
-      if (b->seen[i] != b->members[i]->plan_version)
+      if (b->seen[i] != b->members[i]->plan_version ||
+          (b->active[i] && !cells_in(b->members[i], b->par[i])))
          need = true;
    if (!need)
       return AMR_OK;
@@ -563,8 +576,10 @@ int ensure_table(amr_batch *b)
          BHIP(b, hipGetLastError());
       }
    BHIP(b, hipStreamSynchronize(b->stream));
-   for (size_t i = 0; i < b->members.size(); i++)
+   for (size_t i = 0; i < b->members.size(); i++) {
       b->seen[i] = b->members[i]->plan_version;
+      b->par[i] = b->members[i]->par[0];
+   }
    b->table_ok = true;
    b->table_vpw = b->vpw;
    b->table_wg = b->wg_mask;
@@ -896,6 +911,7 @@ int amr_batch_add(amr_batch *b, const amr_dev_config *cfg, amr_dev **member)
    b->members.push_back(d);
    b->active.push_back(1);
    b->seen.push_back(-1);
+   b->par.push_back(0);
    b->table_ok = false;
    *member = d;
    return AMR_OK;

@@ -90,3 +90,45 @@ def test_wavefront_exchange_items(exchange_vars):
         b.check("wavefront items")
     finally:
         b.close()
+
+
+@pytest.mark.parametrize("st", [7, 27])
+def test_members_cells_in_the_other_copy(st):
+    """The batch steps a member's present cells after calls that left them in
+    the other interior copy: an odd number of fused stages, of all variables
+    and of one, and a saved state."""
+    print("case: batch, members moved between timesteps, stencil %d" % st, flush=True)
+    rng = np.random.default_rng(st)
+    b = Batch(st)
+    try:
+        for n, nv in (((4, 6, 8), 3), ((8, 8, 8), 2)):
+            pair = b.add(n, nv, 12)
+            fill(rng, pair, 12)
+            plan = meshgen.random_plan(rng, 5, 6)
+            for d in pair:
+                d.set_mesh(range(11), plan)
+        m, c = b.pairs[0]
+        b.timestep(0, 2)
+        for k in range(3):
+            m.stage_fused(0, 3, stage=k)
+            c.stage(0, 3, stage=k)
+        b.timestep(2, 2)
+        m.stage_fused(1, 1)
+        c.stage(1, 1)
+        b.timestep(4, 2)
+        b.timestep(6, 2)
+        for d in (m, c):
+            d.stage_fused(0, 3)
+        b.timestep(8, 1)
+        b.check("stages of a member")
+        for d in (m, c):
+            d.stage_fused(0, 3)
+        b.timestep(10, 2)                       # the member now steps from the other copy
+        size = ctypes.c_size_t()
+        assert b.lib.amr_dev_state_bytes(m.h, ctypes.byref(size)) == 0
+        state = np.empty(size.value, dtype=np.uint8)
+        assert b.lib.amr_dev_save_state(m.h, state.ctypes.data_as(ctypes.c_void_p)) == 0
+        b.timestep(12, 2)
+        b.check("a saved state")
+    finally:
+        b.close()
