@@ -461,7 +461,9 @@ int ensure_table(amr_batch *b)
       m.fjobs = d->d_fjobs;
       m.redir = d->d_redir;
       m.edges = d->d_edges;
-      fusable = fusable && d->two_interiors && !d->whole_ghosts && d->g.stencil != 0 &&
+      // closed: jobs that read slots outside the active list find their cells
+      // in one copy only, so such a plan's stages are plain ones
+      fusable = fusable && d->two_interiors && d->closed && !d->whole_ghosts && d->g.stencil != 0 &&
                 !(d->tape && d->tape->on) && (d->d_fjobs || !(d->fcount[0] + d->fcount[1] +
                                                               d->fcount[2])) &&
                 d->d_redir && d->d_edges;

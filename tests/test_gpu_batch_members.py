@@ -132,3 +132,23 @@ def test_members_cells_in_the_other_copy(st):
         b.check("a saved state")
     finally:
         b.close()
+
+
+@pytest.mark.parametrize("st", [7, 27])
+def test_members_plan_reads_inactive_slots(st):
+    """A member whose jobs read slots outside its active list: those cells stay
+    where they are, in every stage of a timestep."""
+    print("case: batch, inactive sources, stencil %d" % st, flush=True)
+    rng = np.random.default_rng(st)
+    b = Batch(st)
+    try:
+        for n, nv in (((4, 6, 8), 3), ((8, 8, 8), 2)):
+            pair = b.add(n, nv, 12)
+            fill(rng, pair, 12)
+            plan = meshgen.random_plan(rng, 5, 6)
+            for d in pair:
+                d.set_mesh(range(5 if nv == 3 else 0, 11), plan)
+        b.timestep(0, 4)
+        b.check("inactive sources")
+    finally:
+        b.close()
