@@ -459,6 +459,16 @@ constexpr int kSpanExchangeX = 4;
 int amr_set_mesh_impl(amr_dev *d, const int32_t *sorted, int n_active, const amr_face_job *jobs,
                       const int32_t count[3]);
 int amr_comm_impl(amr_dev *d, int start, int num, int stage, int permute);
+// An exchange in this order copies ghost cells as the stage before left them
+// into cells that no later phase writes: a 27-point same-level fill takes its
+// source's x- or y-extended rows, and with y or z before x those are last
+// stage's.  (In the order x, y, z -- also the first of the permuted ones --
+// every such copy is written over by a later phase.)  Planes that a fused
+// stage left unwritten have to be brought up to date before.
+inline bool amr_order_reads_ghosts(int stencil, int stage, int permute)
+{
+   return stencil == 27 && permute && stage % 6 != 0;
+}
 int amr_stencil_impl(amr_dev *d, int var, int calc_stage);
 int amr_stage_impl(amr_dev *d, int start, int num, int stage, int permute, int sum_row);
 int amr_split_impl(amr_dev *d, const amr_split_job *jobs, int n);

@@ -770,6 +770,19 @@ void mark_stale(amr_batch *b, bool stale)
          std::fill(b->members[i]->stale.begin(), b->members[i]->stale.end(), stale ? 1 : 0);
 }
 
+// Before a stage that copies ghost cells of the stage before: the members'
+// stale planes.
+int fresh_members(amr_batch *b, int stage, int permute)
+{
+   if (!amr_order_reads_ghosts(b->stencil, stage, permute))
+      return AMR_OK;
+   for (size_t i = 0; i < b->members.size(); i++)
+      if (b->active[i])
+         if (int rc = amr_require_fresh(b->members[i], 0, b->members[i]->c.num_vars, "stage"))
+            return berr(b, rc, "member %d: %s", (int) i, b->members[i]->err);
+   return AMR_OK;
+}
+
 int check_row(amr_batch *b, int row)
 {
    if (row < 0)
@@ -974,6 +987,8 @@ int amr_batch_stage(amr_batch *b, int stage, int permute, int sum_row)
    if (!rc)
       rc = check_row(b, sum_row);
    if (!rc)
+      rc = fresh_members(b, stage, permute);
+   if (!rc)
       rc = enqueue_stage(b, stage, permute, sum_row);
    if (!rc)
       mark_stale(b, false);   // a plain stage writes every ghost plane
@@ -990,6 +1005,8 @@ int amr_batch_timestep(amr_batch *b, int stage0, int nstages, int checksum_freq,
    if (rc)
       return rc;
    if (checksum_freq && (rc = check_row(b, (nstages - 1) / checksum_freq)))
+      return rc;
+   if ((rc = fresh_members(b, stage0, permute)))
       return rc;
    const bool fused = fuse_timestep(b, nstages, permute);
    const long key[11] = {b->epoch, permute ? stage0 % 6 : -1, nstages, checksum_freq,

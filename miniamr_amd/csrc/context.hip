@@ -1093,6 +1093,9 @@ int amr_comm_impl(amr_dev *d, int start, int num, int stage, int permute)
                            start + num);
    if (!num)
       return AMR_OK;
+   if (amr_order_reads_ghosts(d->g.stencil, stage, permute))
+      if (int rc = amr_require_fresh(d, start, num, "comm"))
+         return rc;
    if (int rc = amr_unify(d, start, num))
       return rc;
    // one span per direction when timing per direction, else one in all

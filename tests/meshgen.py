@@ -78,3 +78,23 @@ def merge_jobs_with_reuse(rng, n_merges):
         for o, c in enumerate(kids):
             jobs.append((dst, c, o, 0))
     return np.array(jobs, dtype=MERGE_JOB)
+
+
+def box_plan(bx, by, bz):
+    """A uniform box of bx x by x bz blocks in slots [0, bx*by*bz): same-level
+    jobs between neighbours, boundary fills at the box's faces.  Returns the
+    slots and the jobs of the three directions."""
+    dims = (bx, by, bz)
+    slot = np.arange(bx * by * bz).reshape(dims)
+    by_dir = []
+    for d in range(3):
+        jobs = []
+        for at in np.ndindex(*dims):
+            for hi in range(2):
+                nb = list(at)
+                nb[d] += 2 * hi - 1
+                inside = 0 <= nb[d] < dims[d]
+                jobs.append((FACE_SAME if inside else FACE_BC, 2 * d + hi, slot[at],
+                             slot[tuple(nb)] if inside else slot[at], 0, 0))
+        by_dir.append(np.array(jobs, dtype=FACE_JOB))
+    return list(range(bx * by * bz)), by_dir

@@ -152,3 +152,30 @@ def test_members_plan_reads_inactive_slots(st):
         b.check("inactive sources")
     finally:
         b.close()
+
+
+@pytest.mark.parametrize("st", [7, 27])
+def test_permuted_stages_after_fused_timesteps(st):
+    """Permuted stages copy ghost cells that the stage before wrote; a fused
+    timestep leaves them unwritten."""
+    print("case: batch, permuted after fused, stencil %d" % st, flush=True)
+    rng = np.random.default_rng(st)
+    b = Batch(st)
+    try:
+        for n, box in (((4, 6, 8), (3, 2, 2)), ((8, 8, 8), (2, 1, 3))):
+            order, plan = meshgen.box_plan(*box)
+            pair = b.add(n, 2, len(order))
+            fill(rng, pair, len(order))
+            for d in pair:
+                d.set_mesh(order, plan)
+        for k in range(1, 6):
+            b.timestep(0, 2)
+            if k % 2:
+                b.timestep(k, 1, permute=True)
+            else:
+                b.ok(b.lib.amr_batch_stage(b.h, k, 1, -1))
+                for _, c in b.pairs:
+                    c.stage(0, 2, stage=k, permute=True)
+            b.check("permutation %d" % k)
+    finally:
+        b.close()

@@ -130,3 +130,24 @@ def test_compare_cells_while_variables_are_in_different_copies():
     assert g.lib.amr_dev_compare_cells(g.h, c.h, 0, NV, worst) == 0
     assert list(worst) == [0.0] * NV
     same(g, c)
+
+
+@pytest.mark.parametrize("what", ["stage", "comm"])
+@pytest.mark.parametrize("st", [7, 27])
+def test_permuted_exchange_after_fused_stages(st, what):
+    """With y or z first, a 27-point exchange copies ghost cells that the stage
+    before wrote: after a fused stage they are brought up to date first.  Every
+    block of a box is its neighbours' source, the domain boundary included."""
+    print("case: permuted exchange after fused stages, %s, stencil %d" % (what, st), flush=True)
+    g, c, _ = pair(st)
+    order, plan = meshgen.box_plan(3, 2, 2)
+    for d in (g, c):
+        d.set_mesh(order, plan)
+    for k in range(6):
+        stages(g, c, 0, NV, 0, 1 + k % 2)
+        if what == "comm":
+            g.comm(0, NV, stage=k, permute=True)
+            c.comm(0, NV, stage=k, permute=True)
+        else:
+            stages(g, c, 0, NV, k, 1, permute=True)
+        same(g, c, order)
