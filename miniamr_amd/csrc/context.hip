@@ -235,6 +235,8 @@ int amr_dev_upload_block(amr_dev *d, int slot, const double *cells)
 {
    if (!d || !cells || slot < 0 || slot >= d->c.max_blocks)
       return amr_set_error(d, AMR_ERR_ARG, "upload: slot %d out of range", slot);
+   if (amr_require_fresh(d, 0, d->c.num_vars, "upload_block"))   // or later: over these cells
+      return AMR_ERR_STATE;
    if (int rc = amr_unify(d, 0, d->c.num_vars))
       return rc;
    size_t bytes = sizeof(double) * (size_t) d->g.gx * d->g.gy * d->g.gz * d->c.num_vars;

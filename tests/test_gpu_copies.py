@@ -151,3 +151,26 @@ def test_permuted_exchange_after_fused_stages(st, what):
         else:
             stages(g, c, 0, NV, k, 1, permute=True)
         same(g, c, order)
+
+
+@pytest.mark.parametrize("st", [7, 27])
+def test_upload_after_fused_stages(st):
+    """An upload's ghost cells stay as uploaded, and the stencil reads them."""
+    print("case: upload after fused stages, stencil %d" % st, flush=True)
+    g, c, rng = pair(st)
+    plan = meshgen.random_plan(rng, 5, 6)
+    for d in (g, c):
+        d.set_mesh(range(11), plan)
+    stages(g, c, 0, NV, 0, 3)
+    for s in (2, 7, 10):
+        cells = rng.random(g.shape)
+        for d in (g, c):
+            d.upload(s, cells)
+    same(g, c)
+    stages(g, c, 0, NV, 3)
+    cells = rng.random(g.shape)
+    for d in (g, c):
+        d.upload(8, cells)
+        for v in range(NV):
+            d.stencil(v)
+    same(g, c)
