@@ -1020,6 +1020,10 @@ int amr_dev_clear_block(amr_dev *d, int slot)
 {
    if (!d || slot < 0 || slot >= d->c.max_blocks)
       return amr_set_error(d, AMR_ERR_ARG, "clear_block: slot %d out of range", slot);
+   // both copies of the slot's cells go: planes that are still to be filled
+   // from them, and its own, are filled before
+   if (amr_require_fresh(d, 0, d->c.num_vars, "clear_block"))
+      return AMR_ERR_STATE;
    return by_precision(d->c.precision, [&](auto z) -> int {
       typedef decltype(z) T;
       hipLaunchKernelGGL(k_clear_slot<T>, dim3((unsigned) ((d->g.rec + 255) / 256), d->c.num_vars),

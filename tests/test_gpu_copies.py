@@ -174,3 +174,20 @@ def test_upload_after_fused_stages(st):
         for v in range(NV):
             d.stencil(v)
     same(g, c)
+
+
+@pytest.mark.parametrize("st", [7, 27])
+def test_clear_block_after_fused_stages(st):
+    """A cleared slot is zero, ghost planes too, and its neighbours' ghost
+    planes keep the cells they had from it."""
+    print("case: clear_block after fused stages, stencil %d" % st, flush=True)
+    g, c, rng = pair(st, other=M.LIB_PATH)
+    plan = meshgen.random_plan(rng, 5, 6)
+    for d in (g, c):
+        d.set_mesh(range(11), plan)
+    stages(g, c, 0, NV)
+    for s in (1, 2, 3, 8, 20):
+        for d in (g, c):
+            assert d.lib.amr_dev_clear_block(d.h, s) == 0
+    assert not g.download(8).any() and not g.download(20).any()
+    same(g, c)
