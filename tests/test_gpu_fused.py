@@ -1,20 +1,21 @@
-"""Stages that read same-level faces in place (amr_dev_stage_fused).
+"""Stages that read faces in place (amr_dev_stage_fused).
 
 The drop-in driver runs every stage of a timestep as a fused stage but the
-last one before a refinement or the end of the run (by default when a stage
-has >= 1e8 cell updates; MINIAMR_FUSED=2 at every size, as here): the
-stencil reads same-level neighbours'
-interiors instead of ghost copies, writing to the second interior copy of
-each record.  Every checksum and every final cell (ghosts included) must
-be bit-identical to the plain stages' run, on every golden mesh (7- and
-27-point, permuted exchanges -- where the fused stage is the plain one --,
-variable groups, refinement with stale ghosts), and the golden records of
-the reference must still hold.  By default the fused stage also drops the
-27-point edge extensions of the faces it reads in place (the stencil and
-the remaining jobs read those edge cells where the extension would have
-copied them from); the plan that keeps them as jobs is tested too.  A
-context also refuses the calls that need
-written ghost planes until a plain exchange has run.
+last one before a refinement or the end of the run: the stencil reads
+same-level neighbours' and the block's own boundary planes (7-point boxes in
+LDS: coarse and fine neighbours' too) instead of ghost copies, writing to the
+second interior copy of each record.  MINIAMR_FUSED=2, as here, also fuses
+small stages of the plans that fuse from 1e8 cell updates only by default
+(edge extensions kept as jobs, 7-point blocks whose box does not fit).  Every
+checksum and every final cell (ghosts included) must be bit-identical to the
+plain stages' run, on every golden mesh (7- and 27-point, permuted exchanges --
+where a 27-point fused stage is the plain one --, variable groups, refinement
+with stale ghosts), and the golden records of the reference must still hold.
+By default the fused stage also drops the 27-point edge extensions of the faces
+it reads in place (the stencil reads those edge cells where the extension would
+have copied them from); the plan that keeps them as jobs is tested too.  Calls
+that look at ghost planes after fused stages see them as the plain stages
+would have written them.
 """
 import os
 
@@ -28,8 +29,7 @@ from conftest import require
 
 CASES = sorted(f[:-5] for f in os.listdir(A.GOLDEN)
                if f.endswith(".json") and not f.startswith("report_"))
-# "2": fused at every size (by default only stages of >= 1e8 cell updates
-# are); "0": the plain stages
+# "2": fused at every size, whatever the plan; "0": the plain stages
 FUSED = {"MINIAMR_FUSED": "2"}
 
 pytestmark = pytest.mark.gpu
@@ -66,11 +66,16 @@ def assert_same(a, b):
 # in every precision (the ghosts are exact copies), with variable counts
 # that leave partial stencil groups (2, 3, 5 variables against 4 per
 # workgroup) and partial 16-variable exchange items, the bandwidth-scale
-# workload itself (40 variables, fused by default), and the launch-shape
-# overrides.
+# workload itself (40 variables), and the launch-shape overrides.
+# MINIAMR_STENCIL_BOX=0: the plane-by-plane kernels, whose variables per
+# workgroup MINIAMR_STENCIL_VPW sets, in place of the whole-box ones; one mesh
+# takes them at their default shape.
 NARROW = [("t27_a", None), ("t27_cv", None), ("t7_r3", None), ("cfg4", None), ("cfg1", None),
-          ("t27_cv", {"MINIAMR_STENCIL_VPW": "1", "MINIAMR_EXCHANGE": "16,256"}),
-          ("cfg4", {"MINIAMR_STENCIL_VPW": "2", "MINIAMR_EXCHANGE": "4,128"})]
+          ("t27_cv", {"MINIAMR_STENCIL_VPW": "1", "MINIAMR_EXCHANGE": "16,256",
+                      "MINIAMR_STENCIL_BOX": "0"}),
+          ("cfg4", {"MINIAMR_STENCIL_VPW": "2", "MINIAMR_EXCHANGE": "4,128",
+                    "MINIAMR_STENCIL_BOX": "0"}),
+          ("t27_a", {"MINIAMR_STENCIL_BOX": "0"})]
 
 
 @pytest.mark.parametrize("prec", ["f32", "bf16"])
