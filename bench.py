@@ -581,7 +581,7 @@ def main():
                             "of run t // 10), run setup untimed: warmup %d + timed %d = "
                             "%d runs" % (a.warmup, a.steps, r["runs"]),
                    "schedule": a.schedule,
-                   "ghosts": ("same-level faces read in place"
+                   "ghosts": ("same-level and boundary faces read in place"
                               if os.environ.get("MINIAMR_FUSED", "1") != "0" else "plain"),
                    "avg_active_blocks": round(avg_blocks, 1),
                    "cell_var_updates": updates},
@@ -596,8 +596,8 @@ def main():
                                             HBM_PEAK_GBS, 4)
                                       if traffic and launches and stencil_s > 0 else None),
                      "kernel": "k_stencil_v16 (27-point, 16x16 faces; every stage reads "
-                               "same-level faces in place but the last before a refinement "
-                               "or the run's end), %d launches, %.3f ms avg" % (
+                               "same-level and boundary faces in place but the last before a "
+                               "refinement or the run's end), %d launches, %.3f ms avg" % (
                                    launches, stencil_s / max(1, launches) * 1e3),
                      # the practical ceiling on this GPU: a streaming copy
                      # and read (amr_dev_copy_bandwidth, 4 GiB, best of 3),

@@ -253,9 +253,9 @@ int amr_dev_read_sums(amr_dev *dev, int row0, int n_rows, double *out);
 int amr_dev_stage(amr_dev *dev, int start, int num, int stage, int permute,
                   int sum_row);
 
-/* amr_dev_stage with same-level faces read in place (no counterpart in the
- * reference's interface; the drop-in driver uses it for every stage but the
- * last one of a timestep that ends in a refinement or ends the run).
+/* amr_dev_stage with faces read in place (no counterpart in the reference's
+ * interface; the drop-in driver uses it for every stage but the last one of a
+ * timestep that ends in a refinement or ends the run).
  * Cells, checksums and every ghost value a stencil reads are those of
  * amr_dev_stage.  The difference is where they come from: the ghost planes
  * of same-level and boundary faces, and the 27-point edges, are not
@@ -265,9 +265,10 @@ int amr_dev_stage(amr_dev *dev, int start, int num, int stage, int permute,
  * context was created with MINIAMR_FUSED=0 in the environment, which costs
  * ~70% more pool memory at 16^3).  Those ghost cells are stale until the
  * next amr_dev_stage or amr_dev_comm of the same variables; set_mesh, split,
- * consolidate, stencil, download_block, the halo codec and save_state first
- * bring them up to date (to the values amr_dev_stage would have written,
- * from the interiors the stage read).
+ * consolidate, stencil, upload_block, download_block, clear_block, the halo
+ * codec, save_state and a 27-point exchange in another order than x, y, z
+ * (permute) first bring them up to date (to the values amr_dev_stage would
+ * have written, from the interiors the stage read).
  * With the 7-point stencil every ghost plane -- boundary and coarse/fine ones
  * too -- is read from where its values come from, at any stage size and
  * with permute, where the block's ghost box fits in LDS.  It is

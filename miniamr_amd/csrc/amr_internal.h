@@ -45,8 +45,8 @@ struct Lay {
    int64_t var_stride;      // rec * max_blocks
 };
 
-// A face job of a stage that reads same-level faces in place
-// (amr_dev_stage_fused).  FJ_FULL fills the job's ghost cells as the plain
+// A face job of a stage that reads faces in place (amr_dev_stage_fused; edges
+// folded, only coarse/fine jobs are left).  FJ_FULL fills the job's ghost cells as the plain
 // exchange does; FJ_EXT_ONLY (a same-level y or z face whose face interior
 // the stencil reads from the neighbour directly) fills only the cells
 // outside the face interior: the 27-point edge extension.  alt[] redirects
@@ -194,8 +194,9 @@ struct amr_dev {
    // The plan of amr_dev_stage_fused, derived from the plain plan by
    // set_mesh: reduced job lists per direction, and per active block
    // (sorted order) the slots its six faces are read from in place (-1:
-   // its own ghost plane; kRedirBc: its own plane next to the boundary).  stale[v]: variable v's in-place faces' ghost
-   // planes have not been written since the last plain exchange.
+   // its own ghost plane; kRedirBc: its own plane next to the boundary).
+   // stale[v]: variable v's in-place faces' ghost planes have not been written
+   // since the last plain exchange.
    FusedJob *d_fjobs = nullptr;
    int32_t fcount[3] = {0, 0, 0};
    int fjobs_cap = 0;
@@ -519,8 +520,7 @@ int amr_launch_box(amr_dev *d, int st, const FaceSrc *faces, const EdgeSrc *edge
                    const Lay &Lo, int start, int num, double *parts);
 int amr_launch_mat_stencil(amr_dev *d, int var, int calc_stage);
 // Stencil of a fused stage: interiors read from the current copy, written
-// to the other one (the variables' copy flips), same-level faces read in
-// place.
+// to the other one (the variables' copy flips), faces read in place.
 int amr_launch_stencil_fused(amr_dev *d, int start, int num, bool want_partials);
 // Brings the ghost planes of variables [start, start+num) that an
 // amr_dev_stage_fused left unwritten (stale) up to date: they are set to what

@@ -225,7 +225,8 @@ template <> struct Cls<5> { enum { NC = 4, NP = 6, NZ = 0, D = 4 }; };
 // An item's layout is its member's (a scalar load: the member index is
 // uniform across the item's threads).
 // FUSED: the stencil of a fused stage, reading the copy `flip` names and
-// same-level faces in place, writing the other copy (as k_stencil_fused).
+// same-level and (27-point, edges folded) boundary faces in place, writing the
+// other copy (as k_stencil_fused).
 template <typename T, int ST, int VPW, int C, bool WGM, bool FUSED = false>
 __global__ __launch_bounds__(256) void kb_stencil(const BMember *__restrict__ mem,
                                                   const BStItem *__restrict__ items, int total,

@@ -73,7 +73,7 @@ bool box_dims(const Lay &g, int st, int n_active, int num, BoxDims &B, int &C, i
    if (!QV || bytes > 56 * 1024)
       return false;
    // Variables per workgroup: sweeps as long as 4096 workgroups remain (10^3
-   // FP64, 680 blocks x 40 variables: 94.8 ms a run, 93.8 with 8192, 106.2
+   // FP64, 890 blocks x 40 variables: 94.8 ms a run, 93.8 with 8192, 106.2
    // with one variable each; 16^3 FP32: 129.0 / 130.8 / 147.0).
    const int64_t items = (int64_t) n_active * num;
    int V = (int) std::max<int64_t>(1, std::min<int64_t>(num, items / 4096));

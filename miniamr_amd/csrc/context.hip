@@ -440,8 +440,8 @@ int amr_home_copies(amr_dev *d)
 }
 
 // MINIAMR_HOIST=0 keeps every fused job in its own direction's launch (the
-// default moves the y and z coarse/fine jobs of blocks without a boundary
-// face into the first launch, below).
+// default moves the y and z coarse/fine jobs -- with the edges not folded those
+// of blocks without a boundary face -- into the first launch, below).
 static bool hoist_on()
 {
    static int v = -1;

@@ -2,8 +2,10 @@
 // in LDS.  A workgroup owns one block and sweeps over its variables: each
 // variable's interior and ghost planes are loaded as vectors of C cells in
 // record order, whatever the block's shape, parked in LDS, and every thread
-// computes its outputs from there while the next variable's loads are in
-// flight.
+// computes its outputs from there.  What hides the loads is the other
+// workgroups of the CU: the next variable's loads, held in registers during
+// the sums, took 120-176 registers and cost more waves than they gained (10^3
+// FP64 98.5-103.7 ms a run against 94.8).
 //
 // What bounded the plane-by-plane form (kern_stencil.h) off the 16 x 16 faces
 // it was shaped for: one thread per (j, k) column and a barrier per x plane,

@@ -111,8 +111,8 @@ static int ghosts_needed_after_timestep(const amr_run *R)
 }
 
 /* One stage of variables [start, start+number).  Every stage of a
- * timestep but the last reads same-level faces in place (amr_dev_stage_fused:
- * the same cells and checksums); the last is a plain stage where the ghost
+ * timestep but the last reads faces in place (amr_dev_stage_fused: the same
+ * cells and checksums); the last is a plain stage where the ghost
  * planes are looked at after it (ghosts_needed_after_timestep), so that
  * there every ghost plane holds what the reference's would. */
 static void enqueue_stage(amr_run *R, int start, int number, int stage, int comm_stage,
