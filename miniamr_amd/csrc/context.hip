@@ -69,7 +69,9 @@ void amr_span_end(amr_dev *d)
 // null (pageable memory, device memory, or a range that one allocation does
 // not hold).  A download writes there with its own kernel: staging the block
 // on the device and copying it cost a second launch and pass (3-32 us of a
-// block's 20-50).
+// block's 20-50).  The runtime reports a range's size in 32 bits, so inside an
+// allocation of 4 GiB or more the answer can be null too; the download is then
+// a staged one.
 static double *device_view(void *p, size_t bytes)
 {
    hipPointerAttribute_t a;

@@ -15,10 +15,11 @@
 // 32-bit offsets that do not change), the LDS traffic and the sums.
 //
 // Measured: 890 blocks of 10^3 x 40 variables, FP64, a 7-point stage 365 us
-// (three exchange launches and the stencil) -> 150 us, bound by its traffic
-// (28.7 KB per block-variable of 16 KB algorithmic: ghost planes, z-plane
-// copies, 80-byte rows in 128-byte lines) and the workgroups in flight; 64
-// blocks of 8^3 x 4 variables 23 -> 5 us, bound by the launch.
+// (three exchange launches and the stencil) -> 152 us, bound by its traffic
+// (22.7 KB per block-variable of 16 KB algorithmic: ghost planes, z-plane
+// copies, 80-byte rows in 128-byte lines; 5.3 TB/s, 0.82 of a copy's rate) and
+// the workgroups in flight; 64 blocks of 8^3 x 4 variables 23 -> 5 us, bound by
+// the launch.
 //
 // Faces.  A ghost plane is read from where its values come from (FaceSrc): the
 // block's own plane, a same-level neighbour's interior, the block's own

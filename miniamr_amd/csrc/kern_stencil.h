@@ -122,13 +122,13 @@ template <typename T> __device__ __forceinline__ T load_at(gptr<T> b, int64_t o)
 //
 // FUSED (a stage that reads same-level and boundary faces in place): the
 // block's slot bslot, redir[6], the slots its six faces are read from (-1: its
-// own ghost plane; kRedirBc: its own plane next to the face), and es[kEdgeSrcs], where its ghost edge lines and corners are
-// read (EdgeSrc).  The face interior of a redirected face is read from the
-// neighbour's interior (its z-plane copy for z faces) in the copy L
-// describes, and the outputs go to the copy Lout describes, so no
-// neighbour's cells change while they are read.  Plane offsets are then
-// 64-bit offsets from the variable's base, the source block varying per
-// element.
+// own ghost plane; kRedirBc: its own plane next to the face), and
+// es[kEdgeSrcs], where its ghost edge lines and corners are read (EdgeSrc).
+// The face interior of a redirected face is read from the neighbour's interior
+// (its z-plane copy for z faces) in the copy L describes, and the outputs go
+// to the copy Lout describes, so no neighbour's cells change while they are
+// read.  Plane offsets are then 64-bit offsets from the variable's base, the
+// source block varying per element.
 template <typename T, int ST, int NCOL, int NPER, int VPW, int NT = kThreads, int NZ = 0,
           int D = kDepth, bool FUSED = false>
 __device__ __forceinline__ void stencil_block(T *__restrict__ rec, const Lay &L, int nv,
